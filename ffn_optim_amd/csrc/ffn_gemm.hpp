@@ -1350,6 +1350,49 @@ struct Engine {
             }
     }
 
+    // The same for a wave holding more blocks, one batch of GB register groups after another: a
+    // batch starts from the own piece (`keep`) or zero and adds the other pieces in K order, the GB
+    // loads of a piece in flight together (~1 us for a device-scope load, whether one or eight are
+    // under way).  Only a batch's registers are carried through its loop over the pieces; with all
+    // of them carried, and no fence between loads and sums, the compiler gave most 16x16 tiles one
+    // load in flight: 16 to 32 dependent round trips per piece.
+    static constexpr int GB = C::WGK == 1 && C::NW == 4 && FN * FM * NQ <= 32 ? 16 : 8;
+    template <int I0, int I1, int B, class Nth, class SlotOf>
+    __device__ __forceinline__ void sum_batches(const __amdgpu_buffer_rsrc_t& r, int first, int last, bool keep,
+                                                int t, const Nth& nth, const SlotOf& slot_of,
+                                                Acc (&acc)[FN][FM]) const {
+        constexpr int RB = I1 - I0, NG = FN * RB * NQ;
+        if constexpr (B * GB < NG) {
+            constexpr int GN = NG - B * GB < GB ? NG - B * GB : GB;
+            f32x4 s[GN];
+#pragma unroll
+            for (int x = 0; x < GN; ++x) {
+                const int g = B * GB + x, j = g / (RB * NQ), i = I0 + (g / NQ) % RB, q = g % NQ;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[x][e] = keep ? acc[j][i][4 * q + e] : 0.0f;
+            }
+            for (int w = nth(first, 0); w <= last; w = nth(w + 1, 0)) {
+                const uint32_t so = slot_of(w);
+                f32x4 v[GN];
+#pragma unroll
+                for (int x = 0; x < GN; ++x) {
+                    const int g = B * GB + x;
+                    v[x] = load_coherent(r, so + part_off(((g / (RB * NQ)) * FM + I0 + (g / NQ) % RB) * NQ + g % NQ, t));
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int x = 0; x < GN; ++x) s[x] += v[x];
+            }
+#pragma unroll
+            for (int x = 0; x < GN; ++x) {
+                const int g = B * GB + x, j = g / (RB * NQ), i = I0 + (g / NQ) % RB, q = g % NQ;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[j][i][4 * q + e] = s[x][e];
+            }
+            sum_batches<I0, I1, B + 1>(r, first, last, keep, t, nth, slot_of, acc);
+        }
+    }
+
     // A Stream-K piece of split tile s, after its partial is stored: the wave counts itself in
     // on the tile's counter for this wave (one counter per wave, since every wave stores and
     // later reduces only the positions it holds), and the wave that arrives last -- its partial
@@ -1386,19 +1429,23 @@ struct Engine {
         constexpr int PC = FN * (I1 - I0) <= 2 ? 4 : 1;
         // k-th piece to add from w0 on (the own piece skipped when kept)
         auto nth = [&](int w0, int k) { return w0 + k + ((keep && w0 <= v && w0 + k >= v) ? 1 : 0); };
-        bool set = !keep;
-        for (int w = first; nth(w, 0) <= last;) {
-            uint32_t so[PC];
-            int c = 0;
+        if constexpr (PC > 1) {
+            bool set = !keep;
+            for (int w = first; nth(w, 0) <= last;) {
+                uint32_t so[PC];
+                int c = 0;
 #pragma unroll
-            for (int k = 0; k < PC; ++k) {
-                const int wk_ = nth(w, k);
-                so[k] = wk_ <= last ? slot_of(wk_) : 0u;
-                c += wk_ <= last ? 1 : 0;
+                for (int k = 0; k < PC; ++k) {
+                    const int wk_ = nth(w, k);
+                    so[k] = wk_ <= last ? slot_of(wk_) : 0u;
+                    c += wk_ <= last ? 1 : 0;
+                }
+                add_pieces<PC, I0, I1>(r, so, c, set, t, acc);
+                set = false;
+                w = nth(w, PC - 1) + 1;
             }
-            add_pieces<PC, I0, I1>(r, so, c, set, t, acc);
-            set = false;
-            w = nth(w, PC - 1) + 1;
+        } else {
+            sum_batches<I0, I1, 0>(r, first, last, keep, t, nth, slot_of, acc);
         }
         store_tile_regs<EPI, I0, I1>(p, u, acc);
     }
