@@ -70,6 +70,7 @@ struct GemmParams {
     int group_m;          // tile-order swizzle: tiles walk group_m tile-rows column by column
     int fast_dma;         // 1: launch the kernel whose interior tiles refill through the SALU-addressed DMA path
     int rev_m;            // 1: tile rows are walked last-first
+    unsigned rot_step;    // tile column tn starts its K range tn * rot_step / 2^16 iterations in (TileCfg::ROT tiles)
     int zero_row0;        // rows [zero_row0, M) of C lie past every tile holding data: written as zeros
     int c_cols;           // columns of C (N, or N / 2 for SwiGLU, whose column pairs make one output)
     const void* bias;     // per-column bias in the storage type, added in FP32 before the activation
@@ -155,6 +156,10 @@ struct TileCfg {
     // after the previous iteration's stage barrier -- the moment the stage they fill is free --
     // instead of in the iteration before the data is used: a full iteration of lead for them.
     static constexpr int EARLY = EARLY_;
+    // Tiles whose units may take their K range rotated (Engine::first_kit): those of small-M GEMMs.
+    // (The wrap's three scalar instructions an iteration would cost the K-sliced 128x128 tile 0.5% on
+    // the aligned mid-size FFN.)
+    static constexpr bool ROT = BM_ <= 64;
     static_assert(EARLY_ == 0 || (STAGES_ == 2 && WGK_ == 1 && EARLY_ < A_PW + B_PW),
                   "early refill: two stages, no K slices, part of the refill");
     static constexpr int LDS_BYTES = STAGES * STAGE_BYTES;
@@ -553,7 +558,18 @@ struct Engine {
         }
         return d;
     }
-    // Per-iteration scalars: the K byte offset of K-iteration kit, and the number of K elements
+    // First K-iteration of a unit.  Tiles with C::ROT may take their range rotated, from a start in
+    // [kb, ke) on and wrapping at ke: tile columns start evenly spread, so that concurrent
+    // workgroups read their weight rows at different offsets (GemmParams::rot_step, 0: in order;
+    // the host divides, which here cost a short launch 1.5%).  Tiles of one column share the start:
+    // their panel of B is fetched once.
+    __device__ __forceinline__ int first_kit(const GemmParams& p, const Unit& u) const {
+        // at most S - 1 short of the end: the DMA prologue then never wraps
+        if constexpr (C::ROT)
+            return u.kb + max(0, min((int)(((unsigned)u.tn * p.rot_step) >> 16), u.ke - u.kb - (S - 1)));
+        else return u.kb;
+    }
+    // Per-iteration scalars: the K byte offset of a unit's iteration, and the number of K elements
     // left from there (0 for an iteration past the unit, whose DMA then reads only zeros).
     struct DmaIt {
         uint32_t k0x2;
@@ -561,8 +577,12 @@ struct Engine {
         uint32_t e_k0x2;  // the same for the iteration whose early refill (C::EARLY) this one issues
         int e_lim;
     };
-    __device__ __forceinline__ DmaIt dma_it(const GemmParams& p, int kit, bool real) const {
+    // kit: the unit's first K-iteration (first_kit) plus the iteration's place in the unit.
+    template <bool WRAP = C::ROT>
+    __device__ __forceinline__ DmaIt dma_it(const GemmParams& p, const Unit& u, int kit, bool real) const {
         DmaIt t{};
+        if constexpr (WRAP)
+            if (kit >= u.ke) kit -= u.ke - u.kb;
         t.k0x2 = (uint32_t)(kit * C::BK * 2);
         t.lim = real ? p.K - kit * C::BK : 0;
         return t;
@@ -656,12 +676,13 @@ struct Engine {
         __amdgpu_buffer_rsrc_t ra, rb;
         rsrc(p, u, ra, rb);
         const DmaLane L = dma_lane(p, u);
+        const int k0 = first_kit(p, u);
 #pragma unroll
         for (int s = 0; s < S - 1; ++s)
-            issue_range<false, 0, C::LOADS>(p, ra, rb, s, L, dma_it(p, u.kb + s, u.kb + s < u.ke));
+            issue_range<false, 0, C::LOADS>(p, ra, rb, s, L, dma_it<false>(p, u, k0 + s, u.kb + s < u.ke));
         // the early part of iteration S-1, whose stage is free too
         if constexpr (C::EARLY > 0)
-            issue_range<false, 0, C::EARLY>(p, ra, rb, S - 1, L, dma_it(p, u.kb + S - 1, u.kb + S - 1 < u.ke));
+            issue_range<false, 0, C::EARLY>(p, ra, rb, S - 1, L, dma_it(p, u, k0 + S - 1, u.kb + S - 1 < u.ke));
     }
     // loads of an issuing wave's DMA prologue (what the next unit has in flight at its start)
     static constexpr int PRO_LOADS = C::LOADS * (S - 1) + C::EARLY;
@@ -879,11 +900,11 @@ struct Engine {
     template <bool FAST>
     __device__ __forceinline__ void step(const GemmParams& p, const Unit& u, const Unit& nx,
                                          const __amdgpu_buffer_rsrc_t& ra, const __amdgpu_buffer_rsrc_t& rb,
-                                         const DmaLane& L, Acc (&acc)[FN][FM], int& cur, int it, int n) {
+                                         const DmaLane& L, Acc (&acc)[FN][FM], int& cur, int it, int n, int k0) {
         const int dkit = it + S - 1;
-        DmaIt o = dma_it(p, u.kb + dkit, FAST || dkit < n);
+        DmaIt o = dma_it(p, u, k0 + dkit, FAST || dkit < n);
         if constexpr (C::EARLY > 0) {
-            const DmaIt e = dma_it(p, u.kb + dkit + 1, dkit + 1 < n);
+            const DmaIt e = dma_it(p, u, k0 + dkit + 1, dkit + 1 < n);
             o.e_k0x2 = e.k0x2, o.e_lim = e.lim;
         }
         const int dstage = (cur == 0) ? S - 1 : cur - 1;
@@ -924,12 +945,15 @@ struct Engine {
         // take the checked one.  (A kernel without FASTK carries the checked loop alone: the
         // second loop body would raise its scalar register pressure.)
         int cur = 0, it = 0;
+        const int k0 = first_kit(p, u);
         if constexpr (FASTK) {
             const bool interior = (u.tm + 1) * C::BM <= p.m_valid && (u.tn + 1) * C::BN <= p.n_valid;
-            const int fast_end = interior ? max(0, min(n, p.K / C::BK - u.kb) - (S - 1)) : 0;
-            for (; it < fast_end && it < n - 1; ++it) step<true>(p, u, nx, ra, rb, L, acc, cur, it, n);
+            const int full = p.K / C::BK - u.kb;  // whole iterations; a rotated K tail may come anywhere
+            const int fast_end =
+                interior && !(C::ROT && k0 != u.kb && full < n) ? max(0, min(n, full) - (S - 1)) : 0;
+            for (; it < fast_end && it < n - 1; ++it) step<true>(p, u, nx, ra, rb, L, acc, cur, it, n, k0);
         }
-        for (; it < n - 1; ++it) step<false>(p, u, nx, ra, rb, L, acc, cur, it, n);
+        for (; it < n - 1; ++it) step<false>(p, u, nx, ra, rb, L, acc, cur, it, n, k0);
         ksteps<false, true, 0>(p, nx, ra, rb, cur, 0, L, DmaIt{0u, 0, 0u, 0}, acc);
     }
 

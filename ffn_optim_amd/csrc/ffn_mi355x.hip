@@ -365,6 +365,26 @@ int group_m_for(long long tiles_m) { return (int)(tiles_m < 4 ? tiles_m : 4); }
 constexpr int kFastDmaMaxK = 8192;
 int fast_dma_for(int k) { return k <= kFastDmaMaxK ? 1 : 0; }
 
+// Rotated K ranges (GemmParams::rot_step).  Workgroups that walk K in step read their weight rows at
+// one K offset at a time; where the row pitch is a multiple of 4 KiB those addresses differ in
+// their high bits alone, and they crowd on some of the memory channels.  Starting every tile
+// column at a place of its own in its K range spreads them.  Weights streamed from HBM, rotated
+// against in step, one run: 16 rows, 4096 -> 16384 -> 4096: up 31.0 -> 25.0 us, split down 32.3 ->
+// 27.8; 16 rows, 8192 x 8192: up 30.3 -> 26.9, down 29.6 -> 26.5; 128 rows, 4096 -> 16384: up 41.2 ->
+// 37.9, down 45.2 -> 42.9.  Pitches that are no such multiple (5120, 13824) and weights that stay in
+// the last-level cache are level or, on the shortest launches, 1% behind: they stay in step.  So do
+// taller problems, whose activation panel is shared in the L2 only while it is in step (4096 rows,
+// 1024 -> 4096: down 30.1 -> 42.6 us rotated).  The rule reads the padded widths, so that operands
+// read in place sum in the same order as their padded copies.
+constexpr int kRotMaxRows = 256;
+constexpr int kRotPitch = 4096;                // bytes
+constexpr long long kRotMinWeights = 64 << 20;  // bytes
+// iterations: of a whole tile, or of the smallest piece of a split one.
+unsigned rot_step(int rows, int padded_k, int padded_n, long long iterations, int tiles_n) {
+    if (rows > kRotMaxRows || (padded_k * 2) % kRotPitch != 0 || 2LL * padded_k * padded_n < kRotMinWeights) return 0;
+    return (unsigned)((iterations << 16) / tiles_n);
+}
+
 // Depth of the down GEMM's reduction: the logical H when hidden rows can be read to it in
 // whole 16-byte chunks, else the padded H (W2 then spans hp columns, zero past h).
 int down_depth(const ffn_mi355x_plan* p) { return p->h % 8 == 0 ? p->h : p->hp; }
@@ -783,6 +803,7 @@ int run_up(const ffn_mi355x_plan* plan, const void* x, const void* w1, const voi
     gp.dp_tiles = gp.tiles_m * gp.tiles_n;
     gp.group_m = group_m_for(gp.tiles_m);
     gp.fast_dma = fast_dma_for(gp.K);
+    gp.rot_step = rot_step(plan->m, plan->kp, gp.N, gp.k_iters, gp.tiles_n);
     gp.bias = b1, gp.bias_n = b1 ? (int)rows : 0;
     if (gather) {
         gp.a_gather = 1;
@@ -803,6 +824,7 @@ int run_up(const ffn_mi355x_plan* plan, const void* x, const void* w1, const voi
         gp.dp_tiles = 0;
         gp.sk_tiles = plan->up_sk_tiles;
         gp.sk_q = (int)(total / plan->up_grid);
+        gp.rot_step = rot_step(plan->m, plan->kp, gp.N, gp.sk_q, gp.tiles_n);
         gp.sk_r = (int)(total % plan->up_grid);
         gp.slots_per_wg = plan->up_slots_per_wg;
         set_workspace(gp, plan, ws, true);
@@ -854,6 +876,7 @@ int run_down(const ffn_mi355x_plan* plan, const void* hidden, const void* w2, co
     gp.k_iters = plan->down_k_iters;
     gp.group_m = group_m_for(gp.tiles_m);
     gp.fast_dma = fast_dma_for(gp.K);
+    gp.rot_step = rot_step(plan->m, plan->hp, gp.N, gp.k_iters, gp.tiles_n);
     // the up GEMM writes hidden tile row after tile row: starting from its last rows finds
     // more of hidden in the last-level cache (DiT-size FFN step: 1044 -> 1037 us Basic,
     // 1056 -> 1043 us Stream-K)
@@ -870,6 +893,7 @@ int run_down(const ffn_mi355x_plan* plan, const void* hidden, const void* w2, co
         gp.sk_tiles = plan->down_sk_tiles;
         const long long total = (long long)plan->down_sk_tiles * plan->down_k_iters;
         gp.sk_q = (int)(total / G);
+        if (gp.dp_tiles == 0) gp.rot_step = rot_step(plan->m, plan->hp, gp.N, gp.sk_q, gp.tiles_n);
         gp.sk_r = (int)(total % G);
         gp.slots_per_wg = plan->down_slots_per_wg;
         set_workspace(gp, plan, ws, false);

@@ -1,0 +1,104 @@
+"""Rotated K ranges and the split Basic down, on integer-valued operands whose sums are exact: every
+result must be the float64 product rounded once, whatever the order of the sum.
+
+Rotation (rows <= 256, a padded depth whose pitch is a multiple of 4 KiB, 64 MiB of weights or more):
+a K tail then lands in the middle of a tile's iterations, and every tile column starts elsewhere.  Split Basic: given a
+workspace the tiles are split along H and finished in the launch; without one they run whole.
+"""
+import ctypes
+import sys
+
+import pytest
+import torch
+
+from ffn_optim_amd import _lib
+from gpu_workspace import counters_are_zero, poisoned_workspace
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*args):
+    print("[split-rotate]", *args, file=sys.stderr, flush=True)
+
+
+def _align(v, unit):
+    return (v + unit - 1) // unit * unit
+
+
+def _operands(m, h, n, hp, np_, dtype, seed):
+    gen = torch.Generator().manual_seed(seed)
+    mp = _align(m, 64)
+    hid = torch.zeros((mp, hp), dtype=dtype)
+    w2 = torch.zeros((np_, hp), dtype=dtype)
+    hid[:m, :h] = torch.randint(-2, 3, (m, h), generator=gen, dtype=torch.int8).to(dtype)
+    w2[:n, :h] = torch.randint(-2, 3, (n, h), generator=gen, dtype=torch.int8).to(dtype)
+    # integer sums below 2^24 are exact in float32
+    golden = torch.zeros((mp, np_), dtype=dtype)
+    golden[:m] = (hid[:m].float() @ w2.float().T).to(dtype)
+    return hid, w2, golden
+
+
+# depths with and without a K tail (2000 = 31 x 64 + 16, 8176 = 63 x 128 + 112)
+@pytest.mark.parametrize("m, h, n, dtype", [
+    (1, 2048, 16384, torch.bfloat16),
+    (16, 8176, 4100, torch.bfloat16),
+    (65, 2000, 16500, torch.float16),
+    (256, 65536, 512, torch.bfloat16),
+    (257, 2048, 16384, torch.float16),   # one row too many: in step
+    (65, 2000, 192, torch.float16),      # too few weights: in step, split
+])
+def test_rotated_down_is_exact_on_all_variants(m, h, n, dtype):
+    lib = _lib.load()
+    hp, np_ = _align(h, 2048), _align(n, 64)
+    hid, w2, golden = _operands(m, h, n, hp, np_, dtype, m)
+    code = _lib.BF16 if dtype == torch.bfloat16 else _lib.FP16
+    hid_d, w2_d = hid.cuda(), w2.cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+    ran = 0
+    for variant in range(lib.ffn_mi355x_num_variants()):
+        for down in ("basic", "streamk"):
+            try:
+                plan = _lib.make_plan(hid.shape[0], 64, hp, np_, code, down, "erf", 256, 0, variant, m=m)
+            except ValueError:
+                continue
+            _lib.set_operands(plan, 64, h, n, 64, 64, hp)
+            for ws in (poisoned_workspace(plan), None):
+                if ws is None and down == "streamk":
+                    continue
+                say(m, h, n, dtype, variant, down, "split" if plan.down_sk_tiles and ws is not None else "whole")
+                out = torch.full(golden.shape, float("nan"), dtype=dtype, device="cuda")
+                _lib.check(lib.ffn_mi355x_down(ctypes.byref(plan), hid_d.data_ptr(), w2_d.data_ptr(), out.data_ptr(),
+                                               ws.data_ptr() if ws is not None else None, stream))
+                torch.cuda.synchronize()
+                assert torch.equal(out.cpu()[:m].view(torch.int16), golden[:m].view(torch.int16)), (variant, down)
+                assert ws is None or counters_are_zero(plan, ws), (variant, down)
+                ran += 1
+    assert ran > 2 * lib.ffn_mi355x_num_variants()
+
+
+@pytest.mark.parametrize("m, k, h", [(16, 2048, 16384), (100, 16368, 2200)])
+def test_rotated_up_matches_gelu(m, k, h):
+    """hidden is the erf GELU of the exact sum, to one unit in the last place (float64 GELU)."""
+    lib = _lib.load()
+    kp, hp = _align(k, 2048), _align(h, 64)
+    x, w1, z = _operands(m, k, h, kp, hp, torch.bfloat16, k)
+    z64 = x[:m].double() @ w1.double().T
+    truth = (0.5 * z64 * torch.special.erfc(-z64 / 2 ** 0.5)).to(torch.bfloat16)
+    xd, wd = x.cuda(), w1.cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def ordinal(bits16):
+        b = bits16.int() & 0xFFFF
+        return torch.where(b >= 0x8000, -(b & 0x7FFF), b)
+
+    for variant in range(lib.ffn_mi355x_num_variants()):
+        plan = _lib.make_plan(x.shape[0], kp, hp, 64, _lib.BF16, "basic", "erf", 256, variant, -1, m=m)
+        _lib.set_operands(plan, k, h, 64, kp, kp, hp)
+        say("up", m, k, h, variant, plan.up_sk_tiles)
+        hidden = torch.full((x.shape[0], hp), float("nan"), dtype=torch.bfloat16, device="cuda")
+        ws = poisoned_workspace(plan)
+        _lib.check(lib.ffn_mi355x_up(ctypes.byref(plan), xd.data_ptr(), wd.data_ptr(), hidden.data_ptr(),
+                                     ws.data_ptr(), stream))
+        torch.cuda.synchronize()
+        ulps = (ordinal(hidden.cpu()[:m].view(torch.int16)) - ordinal(truth.view(torch.int16))).abs()
+        assert int(ulps.max()) <= 1, variant
