@@ -114,8 +114,7 @@ constexpr double kCuMfmaRate = 4.8e12;     // FLOP/s per CU a 256x256 tile susta
 constexpr double kCuLoadRate = 60e9;       // B/s per CU of LDS-DMA alongside MFMA work
 constexpr double kLoadLatency = 0.8e-6;    // s, L2/MALL load latency under load
 constexpr double kHbmRate = 6.5e12;        // B/s sustained HBM read rate
-constexpr double kFinishLatency = 1.2e-6;  // s, one dependent step of a split tile's finish:
-                                           // partial write-through, arrival count, partial reads
+constexpr double kPartialRate = 2.6e12;    // B/s, FP32 partials written through and read back
 constexpr double kUnitOverhead = 2.5e-6;   // s per unit: DMA prologue latency + epilogue
 
 // Relative MFMA efficiency of each macro tile (measured on the FFN shapes, 256x256 = 1): the
@@ -132,9 +131,11 @@ double tile_eff(const Variant& v, bool up = false) {
     const int a = v.bm < v.bn ? v.bm : v.bn, b = v.bm < v.bn ? v.bn : v.bm;
     const double refill = (v.prod > 0 ? 1.03 : 1.0) * (v.mf == 16 ? 1.05 : 1.0);
     // The K-sliced 32x32 decode tile (32x32 wave tiles, one MFMA per k-step and wave) reads the
-    // most fragments per MFMA: 0.15, from the 512x1024 -> 4096 -> 1024 FFN's Basic down, where its
-    // 512 tiles took 30.7 us against 27.0 us for 128 K-sliced 64x64 tiles (one tuning run).
-    if (v.wgk > 1) return refill * (a >= 128 ? (v.nw + v.prod >= 8 ? 0.9 : 0.85) : a >= 64 ? 0.3 : 0.15);
+    // most fragments per MFMA: half the K-sliced 64x64 tile's 0.38 (the 512x1024 -> 4096 -> 1024
+    // FFN's Basic down: 512 tiles of it took 30.7 us against 27.0 us for 128 of 64x64, one tuning
+    // run).  0.38 and 0.19 order the tiles of 32 FFN shapes timed in one run (16 to 4096 rows,
+    // whole and split): the picks average 1% behind the fastest tile; at 0.3 and 0.15, 4%.
+    if (v.wgk > 1) return refill * (a >= 128 ? (v.nw + v.prod >= 8 ? 0.9 : 0.85) : a >= 64 ? 0.38 : 0.19);
     if (a >= 256) return refill * 1.0;
     // 256x192 (16x16 blocks): 0.92 per FLOP of the 256x256 tile, from the DiT-size up at eight
     // tiles per CU (493.5 against 453.0 us at six of 256x256) and its H/8 shard at one wave of
@@ -248,15 +249,18 @@ double cost_streamk(const Variant& v, const SkShape& s, long long m_valid, long 
         it_split = std::max(it, (double)(rows_in_tile(v, m_valid) + v.bn) * v.bk * 2.0 * (double)G / kHbmRate);
     double t = it * (double)dp_waves * s.k_iters + it_split * (double)sk_iters +
                kUnitOverhead * (double)(dp_waves + 1);
-    // shared split tiles: each piece writes its FP32 partial through to memory and counts in;
-    // the last reads the others (several at a time when its waves hold at most two 32x32
-    // blocks, one at a time otherwise) and stores the tile
-    const long long pieces_per_tile = std::min<long long>(G, cdiv(s.k_iters, std::max<long long>(1, s.q)) + 1);
+    // shared split tiles: each piece writes its FP32 partial through to memory and counts in; the
+    // last reads the others and stores the tile.  Few tiles pay the latency of that chain (four
+    // pieces: 2.9 us for 16 KiB tiles, 5.4 for 64, 13.5 for 256; two pieces: 2.0 and 4.2 us for 16
+    // and 64), many the memory traffic of the partials (128 tiles of 256x192 in two pieces: 75 MB
+    // in 31 us; 64 of 256x256 in four: 117 MB in 38-46); pieces that straddle tiles finish two.
+    const long long pieces_per_tile =
+        s.pieces ? s.pieces : std::min<long long>(G, cdiv(s.k_iters, std::max<long long>(1, s.q)) + 1);
     if (s.k_iters > sk_iters) {
-        const double tile_bytes = (double)v.bm * v.bn * 4.0;
-        const long long per_read = (long long)v.bm * v.bn / v.nw <= 2048 ? 4 : 1;
-        t += kFinishLatency * (double)(2 + cdiv(pieces_per_tile - 1, per_read)) +
-             (double)pieces_per_tile * tile_bytes / kCuLoadRate;
+        const double tile_bytes = (double)v.bm * v.bn * 4.0, p = (double)pieces_per_tile;
+        const double latency = 1.0e-6 + 0.4e-6 * p + tile_bytes * (24e-12 + 5e-12 * p);
+        const double traffic = (double)s.sk * (2.0 * p - 1.0) * tile_bytes / kPartialRate;
+        t += std::max(latency * (scattered ? 2.0 : 1.0), traffic);
     }
     const double hbm = (double)(N * K + m_valid * K) * 2.0 / kHbmRate;
     return std::max(t, hbm);
@@ -274,11 +278,43 @@ bool better(double c, const Variant& v, double best_cost, const Variant& best, l
                                      tile_eff(v) > tile_eff(best));
 }
 
+// A GEMM with every tile split along K: open to tiles that would leave at least half of the
+// workgroups idle and a reduction deep enough to split (a decode-size FFN with a narrow H, e.g. one
+// GPU's H/8 share of a 16x5120 -> 13824 FFN, whose few up tiles would stream W1 on a few CUs).
+// Every tile is then cut into p equal pieces (sk_grid); the last piece of a tile to finish sums the
+// partials and stores the tile (the up GEMM's applies the activation).  On that decode shard (54
+// up tiles of 32x32, 4 pieces of 10 iterations on 216 workgroups) the split up takes 8.9 us.
+constexpr int kSplitMinIters = 16;
+bool split_whole(const Variant& v, long long m_valid, long long N, long long K, int G, SkShape& s) {
+    const long long tiles = cdiv(m_valid, v.bm) * cdiv(N, v.bn), k_iters = cdiv(K, v.bk);
+    if (tiles * 2 > G || k_iters < kSplitMinIters) return false;
+    const long long grid = sk_grid(tiles, k_iters, G);
+    if (!sk_shape(v, m_valid, N, K, (int)grid, s) || s.grid != grid || s.dp != 0 || s.sk != tiles) return false;
+    const long long kI = s.k_iters, big = (s.q + 1) * s.r;
+    auto owner = [&](long long x) { return s.q == 0 ? x : x < big ? x / (s.q + 1) : s.r + (x - big) / s.q; };
+    for (long long t = 0; t < tiles; ++t)
+        if (owner(t * kI) == owner(t * kI + kI - 1)) return false;
+    return true;
+}
+
+// A Basic down splits its tiles the same way where the model prices that below whole tiles, and
+// the pieces cut a tile's iterations evenly.  Whole tiles left CUs idle on small-M FFNs, whose
+// output is few tiles wide: 128x4096 -> 16384 -> 4096, 128 tiles of 64x64 whole 71.3 us, split in
+// two 46.1, 64 of 64x128 split in four 45.2; 256 rows 71.3 -> 57.2; 512 rows 106.8 (64x128 whole) ->
+// 81.9 (256x128 split); 512x1024 -> 4096 -> 1024, 13.3 -> 11.2.
+bool split_down(const Variant& v, long long M, long long m_valid, long long N, long long K, int G, SkShape& s) {
+    return split_whole(v, m_valid, N, K, G, s) && s.k_iters % s.pieces == 0 &&
+           cost_streamk(v, s, m_valid, N, K) < cost_basic(v, M, m_valid, N, K, G);
+}
+
 int pick_basic(long long M, long long m_valid, long long N, long long K, int G) {
     int best = 0;
     double best_cost = 1e300;
     for (int i = 0; i < kNumVariants; ++i) {
-        const double c = cost_basic(kVariants[i], M, m_valid, N, K, G);
+        SkShape s;
+        const double c = split_down(kVariants[i], M, m_valid, N, K, G, s)
+                             ? cost_streamk(kVariants[i], s, m_valid, N, K)
+                             : cost_basic(kVariants[i], M, m_valid, N, K, G);
         if (better(c, kVariants[i], best_cost, kVariants[best], m_valid)) best_cost = c, best = i;
     }
     return best;
@@ -303,25 +339,6 @@ int pick_streamk(long long M, long long m_valid, long long N, long long K, int G
     return best;
 }
 
-// Split up GEMM: taken when the up's tiles would leave at least half of the workgroups idle and
-// the reduction is deep enough to split (a decode-size FFN with a narrow H, e.g. one GPU's H/8
-// share of a 16x5120 -> 13824 FFN, whose few tiles would stream W1 on a few CUs).  Every tile is
-// then cut into p equal pieces (sk_grid); the last piece of a tile to finish sums the partials
-// and applies the activation.  On that decode shard (54 tiles of 32x32, 4 pieces of 10
-// iterations on 216 workgroups) the split up takes 10.6-10.8 us.
-constexpr int kUpSplitMinIters = 16;
-bool split_up(const Variant& v, long long m_valid, long long N, long long K, int G, SkShape& s) {
-    const long long tiles = cdiv(m_valid, v.bm) * cdiv(N, v.bn), k_iters = cdiv(K, v.bk);
-    if (tiles * 2 > G || k_iters < kUpSplitMinIters) return false;
-    const long long grid = sk_grid(tiles, k_iters, G);
-    if (!sk_shape(v, m_valid, N, K, (int)grid, s) || s.grid != grid || s.dp != 0 || s.sk != tiles) return false;
-    const long long kI = s.k_iters, big = (s.q + 1) * s.r;
-    auto owner = [&](long long x) { return s.q == 0 ? x : x < big ? x / (s.q + 1) : s.r + (x - big) / s.q; };
-    for (long long t = 0; t < tiles; ++t)
-        if (owner(t * kI) == owner(t * kI + kI - 1)) return false;
-    return true;
-}
-
 // Up-GEMM tile when none is forced: every variant is priced as the plan it would get, split
 // along K (Stream-K cost, the finish of split tiles included) or one workgroup per tile.
 // A SwiGLU up GEMM (N = 2 x the hidden width, gate and up rows interleaved in 32-row blocks)
@@ -343,7 +360,7 @@ int pick_up(long long M, long long m_valid, long long N, long long K, int G, boo
     for (int i = 0; i < kNumVariants; ++i) {
         if (swiglu && !swiglu_tile(kVariants[i])) continue;
         SkShape s;
-        const bool split = !swiglu && split_up(kVariants[i], m_valid, N, K, G, s);
+        const bool split = !swiglu && split_whole(kVariants[i], m_valid, N, K, G, s);
         if (split && fills) continue;
         const double c = split ? cost_streamk(kVariants[i], s, m_valid, N, K, true)
                                : cost_basic(kVariants[i], M, m_valid, N, K, G, true);
@@ -500,14 +517,23 @@ constexpr int kSplitWords = FFN_MI355X_SPLIT_COUNTER_WORDS;
 bool spread_counters(long long up_sk, long long down_sk) {
     return (up_sk + down_sk) * kSplitWords <= (long long)(kCounterBytes / 4);
 }
-long long down_split_tiles(const ffn_mi355x_plan* p) {
-    return p->down_impl == FFN_MI355X_DOWN_STREAMK ? p->down_sk_tiles : 0;
-}
+long long down_split_tiles(const ffn_mi355x_plan* p) { return p->down_sk_tiles; }
 int counter_stride(const ffn_mi355x_plan* p, const Variant& v) {
     return spread_counters(p->up_sk_tiles, down_split_tiles(p)) ? kSplitWords : v.nw;
 }
 size_t down_counter_words(const ffn_mi355x_plan* p) {
     return (size_t)down_split_tiles(p) * (size_t)counter_stride(p, kVariants[p->down_variant]);
+}
+// Partial slots of a split up GEMM.
+size_t up_partial_bytes(const ffn_mi355x_plan* p) {
+    return p->up_sk_tiles > 0 ? (size_t)p->up_grid * p->up_slots_per_wg * p->up_bm * p->up_bn * 4u : 0;
+}
+// Workspace of ffn_mi355x_run_noalloc: a Basic down runs whole tiles there, so that Basic plans
+// without a split up GEMM or a single launch share no scratch between overlapping calls.
+size_t noalloc_bytes(const ffn_mi355x_plan* p) {
+    if (p->down_impl == FFN_MI355X_DOWN_STREAMK || p->down_sk_tiles == 0) return p->workspace_bytes;
+    const size_t up = up_partial_bytes(p);
+    return up > 0 || p->single_launch ? up + kCounterBytes : 0;
 }
 size_t up_counter_words(const ffn_mi355x_plan* p) {
     return p->up_sk_tiles > 0 ? (size_t)p->up_sk_tiles * (size_t)counter_stride(p, kVariants[p->up_variant]) : 0;
@@ -607,7 +633,7 @@ int ffn_mi355x_make_plan(int m, int mp, int kp, int hp, int np, int dtype, int d
     plan->up_k_iters = (int)cdiv(kp, U.bk);
     size_t up_ws = 0;
     SkShape su;
-    if (!swiglu && split_up(U, m, hp, kp, G, su)) {
+    if (!swiglu && split_whole(U, m, hp, kp, G, su)) {
         plan->up_sk_tiles = (int)su.sk;
         plan->up_slots_per_wg = (int)su.slots;
         plan->up_grid = (int)su.grid;
@@ -616,6 +642,8 @@ int ffn_mi355x_make_plan(int m, int mp, int kp, int hp, int np, int dtype, int d
 
     // down: [mp x np], depth hp
     int dv;
+    bool split_basic = false;
+    SkShape sb;
     if (down_impl == FFN_MI355X_DOWN_STREAMK) {
         if (down_variant >= 0) {
             SkShape s;
@@ -645,15 +673,16 @@ int ffn_mi355x_make_plan(int m, int mp, int kp, int hp, int np, int dtype, int d
         }
     } else {
         dv = down_variant >= 0 ? down_variant : pick_basic(mp, m, np, hp, G);
+        split_basic = split_down(kVariants[dv], mp, m, np, hp, G, sb);
     }
     const Variant& D = kVariants[dv];
     plan->down_variant = dv;
     plan->down_bm = D.bm, plan->down_bn = D.bn, plan->down_bk = D.bk;
     plan->down_tiles = (int)(cdiv(m, D.bm) * cdiv(np, D.bn));
     plan->down_k_iters = (int)cdiv(hp, D.bk);
-    if (down_impl == FFN_MI355X_DOWN_STREAMK) {
-        SkShape s;
-        sk_shape(D, m, np, hp, G, s);
+    if (down_impl == FFN_MI355X_DOWN_STREAMK || split_basic) {
+        SkShape s = sb;
+        if (!split_basic) sk_shape(D, m, np, hp, G, s);
         plan->down_dp_tiles = (int)s.dp;
         plan->down_sk_tiles = (int)s.sk;
         plan->down_slots_per_wg = (int)s.slots;
@@ -853,13 +882,14 @@ int run_down(const ffn_mi355x_plan* plan, const void* hidden, const void* w2, co
     if (!aligned16(hidden) || !aligned16(w2) || !aligned16(out) || (ws && !aligned16(ws)) || (b2 && !aligned16(b2)))
         return fail(FFN_MI355X_EINVAL, "device buffers must be 16-byte aligned");
     int rc;
+    const bool split = plan->down_impl == FFN_MI355X_DOWN_STREAMK ||
+                       (plan->down_sk_tiles > 0 && ws && !ws_scratch && !built);
     if ((rc = check_span("hidden", hidden, span_bytes(plan->m, plan->hp, down_depth(plan)))) != FFN_MI355X_OK ||
         (rc = check_span("w2", w2, span_bytes(plan->n, plan->ldw2, down_depth(plan)))) != FFN_MI355X_OK ||
         (b2 && (rc = check_span("bias2", b2, (size_t)plan->n * 2u)) != FFN_MI355X_OK) ||
         (rc = check_span("out", out, span_bytes(plan->mp, plan->np, plan->np))) != FFN_MI355X_OK ||
-        (plan->down_impl == FFN_MI355X_DOWN_STREAMK && ws && !ws_scratch &&
-         (rc = check_span("ws", ws, plan->workspace_bytes)) != FFN_MI355X_OK) ||
-        (plan->down_impl != FFN_MI355X_DOWN_STREAMK && ws && !ws_scratch && up_counter_words(plan) > 0 &&
+        (split && ws && !ws_scratch && (rc = check_span("ws", ws, plan->workspace_bytes)) != FFN_MI355X_OK) ||
+        (!split && ws && !ws_scratch && up_counter_words(plan) > 0 &&
          (rc = check_span("ws", ws, flags_bytes(plan))) != FFN_MI355X_OK))
         return rc;
     const Variant& D = kVariants[plan->down_variant];
@@ -886,7 +916,7 @@ int run_down(const ffn_mi355x_plan* plan, const void* hidden, const void* w2, co
         gp.clear_words = up_counters(plan, ws);
         gp.clear_count = (int)up_counter_words(plan);
     }
-    if (plan->down_impl == FFN_MI355X_DOWN_STREAMK) {
+    if (split) {
         if (!ws) return fail(FFN_MI355X_EINVAL, "Stream-K needs a workspace of %zu bytes", plan->workspace_bytes);
         const int G = plan->down_grid;
         gp.dp_tiles = plan->down_dp_tiles;
@@ -904,7 +934,7 @@ int run_down(const ffn_mi355x_plan* plan, const void* hidden, const void* w2, co
         *built = gp;
         return ok();
     }
-    return launch(D, plan->dtype, FFN_ROLE_DOWN_BASIC, gp, plan->down_grid, hip_stream);
+    return launch(D, plan->dtype, FFN_ROLE_DOWN_BASIC, gp, std::min(plan->down_tiles, plan->block_num), hip_stream);
 }
 
 // The whole FFN of a plan: one launch when the plan says so and X is not read as gathered rows
@@ -1014,13 +1044,13 @@ int ffn_mi355x_run_ex(const ffn_mi355x_plan* plan, const void* x, const void* w1
 int ffn_mi355x_run_noalloc(const ffn_mi355x_plan* plan, const void* x, const void* w1, const void* w2,
                            void* hidden, void* out, void* hip_stream) {
     if (!valid_plan(plan)) return fail(FFN_MI355X_EINVAL, "invalid plan");
-    if (plan->workspace_bytes > (size_t)FFN_MI355X_NOALLOC_SCRATCH_BYTES)
+    if (noalloc_bytes(plan) > (size_t)FFN_MI355X_NOALLOC_SCRATCH_BYTES)
         return fail(FFN_MI355X_EINVAL,
                     "plan needs %zu bytes of workspace, more than the %zu bytes of scratch of "
                     "ffn_mi355x_run_noalloc; run it with ffn_mi355x_run and a workspace",
-                    plan->workspace_bytes, (size_t)FFN_MI355X_NOALLOC_SCRATCH_BYTES);
+                    noalloc_bytes(plan), (size_t)FFN_MI355X_NOALLOC_SCRATCH_BYTES);
     void* ws = nullptr;
-    if (plan->workspace_bytes > 0) {
+    if (noalloc_bytes(plan) > 0) {
         const int rc = scratch_address(hip_stream, &ws);
         if (rc != FFN_MI355X_OK) return rc;
     }

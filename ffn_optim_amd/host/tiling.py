@@ -56,8 +56,8 @@ class Plan:
     """Everything one FFN launch sequence needs (reference Plan, tiling.py:28-55).
 
     block_num is the persistent-workgroup count of both launches; mp/kp/hp/np are
-    the padded extents; workspace_shape is the FP32 scratch of the Stream-K down and of
-    a split up GEMM ((1, 1) and unused when neither splits).  native is the C plan handed
+    the padded extents; workspace_shape is the FP32 scratch of a split down (Stream-K, or a
+    small-M Basic) and of a split up GEMM ((1, 1) and unused when neither splits).  native is the C plan handed
     to the library.
 
     workspace_shape keeps the reference's form, FP32 rows of 64 (ops/host/tiling.py:71),
@@ -147,8 +147,8 @@ def make_plan(problem, selection=Selection(), block_num=DEFAULT_BLOCK_NUM, *, ge
                             activation=activation)
     up = _tile(native.up_bm, native.up_bn, native.up_bk, native.up_variant)
     down = _tile(native.down_bm, native.down_bn, native.down_bk, native.down_variant)
-    if native.workspace_bytes:   # Stream-K down and/or split up GEMM
+    if native.workspace_bytes:   # split down and/or split up GEMM
         workspace = (native.workspace_bytes // 256, 64)
     else:
-        workspace = (1, 1)  # unused argument: Basic down, one workgroup per up tile
+        workspace = (1, 1)  # unused argument: one workgroup per up and down tile
     return Plan(problem, selection, block_num, mp, kp, hp, np_, up, down, workspace, gelu, native)

@@ -69,13 +69,15 @@ typedef struct ffn_mi355x_plan {
     int down_bm, down_bn, down_bk; /* down-projection macro tile (M x N x H) */
     int up_tiles, up_grid;
     int down_tiles, down_grid;   /* down_grid <= block_num: fewer for Basic when there are fewer
-                                    tiles, and for Stream-K when that cuts every split tile into
-                                    equal pieces */
+                                    tiles, and for Stream-K or a split Basic down when that cuts
+                                    every split tile into equal pieces */
     int down_k_iters;            /* BK-deep iterations along H per down tile */
     int down_dp_tiles;           /* tiles reduced whole by one workgroup */
-    int down_sk_tiles;           /* tiles whose H-range is split over workgroups */
+    int down_sk_tiles;           /* tiles whose H-range is split over workgroups; a Basic down splits
+                                    all of its tiles or none (whole tiles would leave at least half
+                                    of block_num idle: a small M) */
     int down_slots_per_wg;       /* FP32 partial-tile slots per workgroup */
-    size_t workspace_bytes;      /* FP32 partial-tile slots of the Stream-K down and the split up */
+    size_t workspace_bytes;      /* FP32 partial-tile slots of a split down and the split up */
     /* Operand layout.  ffn_mi355x_make_plan sets the padded buffers (k = kp, h = hp,
        n = np, ldx = ldw1 = kp, ldw2 = hp); ffn_mi355x_set_operands may point the plan at
        operands of their logical widths instead. */
@@ -153,8 +155,9 @@ int ffn_mi355x_set_x_rows(ffn_mi355x_plan* plan, int d1, int d2, int s0, int s1,
  * reference, whose FFN is always one artifact (ops/api.py:43). */
 int ffn_mi355x_set_single_launch(ffn_mi355x_plan* plan, int on);
 
-/* Workspace bytes a plan needs (0 for the Basic down without a split up GEMM or a single
- * launch). */
+/* Workspace bytes a plan uses (0 for a Basic down of whole tiles without a split up GEMM or a
+ * single launch).  A plan whose only use of it is a split Basic down also runs without: see
+ * ffn_mi355x_run. */
 int ffn_mi355x_workspace_bytes(const ffn_mi355x_plan* plan, size_t* bytes);
 
 /* Bytes at the start of every workspace that hold the split tiles' arrival counters (one
@@ -181,9 +184,10 @@ int ffn_mi355x_workspace_counter_bytes(const ffn_mi355x_plan* plan, size_t* byte
  * dtype, then the Basic or Stream-K down GEMM writing `out` [mp,np].  Replaces
  * the single artifact(*tensors, block_num) launch of ops/api.py:43 built by
  * compile_kernel (ops/host/dispatch.py:97-116) from ops/kernel/ffn.py.
- * `ws` must hold plan->workspace_bytes whenever that is nonzero (Stream-K down or
- * split up), its counter bytes as FFN_MI355X_WORKSPACE_COUNTER_BYTES describes; it may be
- * NULL otherwise.
+ * `ws` must hold plan->workspace_bytes for a Stream-K down or a split up, its counter bytes as
+ * FFN_MI355X_WORKSPACE_COUNTER_BYTES describes.  A Basic down splits its tiles (down_sk_tiles)
+ * only when it is given those bytes, and runs whole tiles when `ws` is NULL (the same sums in
+ * another order); without a split GEMM `ws` may be NULL too.
  * The Stream-K down is one launch: the pieces of a split tile store FP32 partial tiles to `ws`,
  * and the last piece to arrive sums them in ascending K order, rounds once and stores the tile.
  * A split up is the same with the GELU applied after the sum. */
@@ -202,7 +206,8 @@ int ffn_mi355x_run(const ffn_mi355x_plan* plan, const void* x, const void* w1,
  * frees nothing.  Every call on one GPU shares that GPU's scratch: calls that overlap on one GPU
  * (on different streams, or from different threads) race and must be serialised by the caller.
  * The scratch starts zero-filled and every call leaves its arrival counters zero again; every
- * partial is written before it is read within a call, so nothing needs clearing. */
+ * partial is written before it is read within a call, so nothing needs clearing.  A Basic down
+ * runs whole tiles here, so a Basic plan without a split up GEMM shares nothing between calls. */
 int ffn_mi355x_run_noalloc(const ffn_mi355x_plan* plan, const void* x, const void* w1,
                            const void* w2, void* hidden, void* out, void* hip_stream);
 
@@ -230,7 +235,7 @@ int ffn_mi355x_up(const ffn_mi355x_plan* plan, const void* x, const void* w1,
                   void* hidden, void* ws, void* hip_stream);
 
 /* Stage 2 alone: Basic (ops/kernel/ffn.py:377-529) or Stream-K
- * (ops/kernel/ffn.py:951-1423) down-projection. */
+ * (ops/kernel/ffn.py:951-1423) down-projection; `ws` as for ffn_mi355x_run. */
 int ffn_mi355x_down(const ffn_mi355x_plan* plan, const void* hidden, const void* w2,
                     void* out, void* ws, void* hip_stream);
 

@@ -102,3 +102,18 @@ def test_rotated_up_matches_gelu(m, k, h):
         torch.cuda.synchronize()
         ulps = (ordinal(hidden.cpu()[:m].view(torch.int16)) - ordinal(truth.view(torch.int16))).abs()
         assert int(ulps.max()) <= 1, variant
+
+
+def test_split_basic_in_place_operands_match_their_copies():
+    """ffn() on operands read in place and the prepared copies run the same split and the same
+    rotated order: bit-identical, and equal on a second call on the same workspace."""
+    from ffn_optim_amd import ffn, prepare_ffn
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn((100, 2040), generator=gen, device="cuda").bfloat16()
+    w1 = (torch.randn((16384, 2040), generator=gen, device="cuda") / 45).bfloat16()
+    w2 = (torch.randn((2100, 16384), generator=gen, device="cuda") / 128).bfloat16()
+    prepared = prepare_ffn(x, w1, w2)
+    assert prepared.plan.native.down_sk_tiles > 0 and prepared.plan.native.down_dp_tiles == 0
+    first = prepared.run().clone()
+    assert torch.equal(first, prepared.run())
+    assert torch.equal(first, ffn(x, w1, w2))

@@ -743,3 +743,28 @@ def test_split_counter_stride_matches_header():
     assert words == _lib.SPLIT_COUNTER_WORDS == 32
     info = _lib.variants()
     assert max(v["waves"] - v["refill_waves"] for v in info) <= words
+
+
+@pytest.mark.parametrize("m, k, h, split", [
+    (128, 4096, 16384, True),      # 128 whole tiles of 64x64 leave half the workgroups idle (71 -> 45 us)
+    (512, 1024, 4096, True),       # (13.3 -> 11.2 us)
+    (16, 5120, 13824, True),       # decode down (33.5 -> 29.3 us)
+    (16, 5120, 1728, False),       # its H/8 shard: 160 whole tiles of 32x32 stay ahead
+    (4096, 1024, 4096, False),     # one whole tile per workgroup
+    (8192, 3072, 12288, False),
+])
+def test_basic_down_splits_only_where_whole_tiles_leave_workgroups_idle(m, k, h, split):
+    """A Basic down splits every tile along H into equal pieces, or none; its workspace then covers
+    the partials.  Every (tile, K-iteration) belongs to one piece and no piece straddles tiles, so
+    each tile is shared by exactly its pieces (the last of which stores it)."""
+    plan = _untuned(m, k, h, "basic")
+    n = plan.native
+    assert (n.down_sk_tiles > 0) == split
+    if not split:
+        assert n.down_sk_tiles == 0 and n.down_dp_tiles == n.down_tiles and n.down_slots_per_wg == 0
+        return
+    assert n.down_sk_tiles == n.down_tiles and n.down_dp_tiles == 0 and 2 * n.down_tiles <= 256
+    pieces, rest = divmod(n.down_grid, n.down_tiles)
+    assert rest == 0 and 2 <= pieces <= 4 and n.down_k_iters % pieces == 0 and n.down_grid <= 256
+    assert n.workspace_bytes >= (_lib.workspace_counter_bytes(n)
+                                 + n.down_grid * n.down_slots_per_wg * n.down_bm * n.down_bn * 4)
