@@ -788,6 +788,14 @@ void set_workspace(ffn::GemmParams& gp, const ffn_mi355x_plan* plan, void* ws, b
     gp.ws_bytes = (unsigned)(plan->workspace_bytes - f);
 }
 
+// Whether a call splits its plan's down GEMM.  A Basic down does so only in a workspace that holds
+// the plan's bytes: with none, a buffer that is too short (Basic plans have not always used one) or
+// the library's scratch it runs whole tiles.
+bool down_is_split(const ffn_mi355x_plan* p, const void* ws, bool ws_scratch) {
+    if (p->down_impl == FFN_MI355X_DOWN_STREAMK) return true;
+    return p->down_sk_tiles > 0 && ws && !ws_scratch && in_allocation(ws, p->workspace_bytes);
+}
+
 // Up GEMM of a plan.  ws_scratch: ws is this library's scratch array (its size is known, and it
 // is not a HIP allocation of its own to look up).
 // Rows of W1 a plan reads: the logical H, or for SwiGLU the 2 hp interleaved gate and up rows.
@@ -806,6 +814,7 @@ int run_up(const ffn_mi355x_plan* plan, const void* x, const void* w1, const voi
         return fail(FFN_MI355X_EINVAL, "the split up GEMM needs a workspace of %zu bytes", plan->workspace_bytes);
     const long long rows = w1_rows(plan);
     int rc;
+    const bool clear_down = ws && down_counter_words(plan) > 0 && down_is_split(plan, ws, ws_scratch);
     const bool gather = plan->x_d1 != 0;
     const size_t x_span = gather ? (size_t)x_grid_span(plan) : span_bytes(plan->m, plan->ldx, plan->k);
     if ((rc = check_span("x", x, x_span)) != FFN_MI355X_OK ||
@@ -813,7 +822,7 @@ int run_up(const ffn_mi355x_plan* plan, const void* x, const void* w1, const voi
         (b1 && (rc = check_span("bias1", b1, (size_t)rows * 2u)) != FFN_MI355X_OK) ||
         (rc = check_span("hidden", hidden, span_bytes(plan->mp, plan->hp, plan->hp))) != FFN_MI355X_OK ||
         (split && !ws_scratch && (rc = check_span("ws", ws, plan->workspace_bytes)) != FFN_MI355X_OK) ||
-        (!split && ws && !ws_scratch && down_counter_words(plan) > 0 &&
+        (!split && !ws_scratch && clear_down &&
          (rc = check_span("ws", ws, flags_bytes(plan))) != FFN_MI355X_OK))
         return rc;
     const Variant& U = kVariants[plan->up_variant];
@@ -840,8 +849,8 @@ int run_up(const ffn_mi355x_plan* plan, const void* x, const void* w1, const voi
         gp.a_s0 = plan->x_s0, gp.a_s1 = plan->x_s1, gp.a_s2 = plan->x_s2;
         gp.a_bytes = (unsigned)x_span;
     }
-    if (ws && down_counter_words(plan) > 0) {
-        // the Stream-K down that follows counts on zero counters: clear them here
+    if (clear_down) {
+        // the split down that follows counts on zero counters: clear them here
         gp.clear_words = (unsigned*)ws;
         gp.clear_count = (int)down_counter_words(plan);
     }
@@ -882,8 +891,7 @@ int run_down(const ffn_mi355x_plan* plan, const void* hidden, const void* w2, co
     if (!aligned16(hidden) || !aligned16(w2) || !aligned16(out) || (ws && !aligned16(ws)) || (b2 && !aligned16(b2)))
         return fail(FFN_MI355X_EINVAL, "device buffers must be 16-byte aligned");
     int rc;
-    const bool split = plan->down_impl == FFN_MI355X_DOWN_STREAMK ||
-                       (plan->down_sk_tiles > 0 && ws && !ws_scratch && !built);
+    const bool split = !built && down_is_split(plan, ws, ws_scratch);
     if ((rc = check_span("hidden", hidden, span_bytes(plan->m, plan->hp, down_depth(plan)))) != FFN_MI355X_OK ||
         (rc = check_span("w2", w2, span_bytes(plan->n, plan->ldw2, down_depth(plan)))) != FFN_MI355X_OK ||
         (b2 && (rc = check_span("bias2", b2, (size_t)plan->n * 2u)) != FFN_MI355X_OK) ||

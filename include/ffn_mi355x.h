@@ -186,8 +186,8 @@ int ffn_mi355x_workspace_counter_bytes(const ffn_mi355x_plan* plan, size_t* byte
  * compile_kernel (ops/host/dispatch.py:97-116) from ops/kernel/ffn.py.
  * `ws` must hold plan->workspace_bytes for a Stream-K down or a split up, its counter bytes as
  * FFN_MI355X_WORKSPACE_COUNTER_BYTES describes.  A Basic down splits its tiles (down_sk_tiles)
- * only when it is given those bytes, and runs whole tiles when `ws` is NULL (the same sums in
- * another order); without a split GEMM `ws` may be NULL too.
+ * only when it is given those bytes, and runs whole tiles when `ws` is NULL or shorter (the same
+ * sums in another order); without a split GEMM `ws` may be NULL too.
  * The Stream-K down is one launch: the pieces of a split tile store FP32 partial tiles to `ws`,
  * and the last piece to arrive sums them in ascending K order, rounds once and stores the tile.
  * A split up is the same with the GELU applied after the sum. */
