@@ -26,6 +26,10 @@ MAX_PITCH = 4_000_000
 SPLIT_COUNTER_WORDS = 32
 
 
+# plans kept by make_plan (a few hundred bytes each)
+MAX_PLANS = 1024
+
+
 class PlanStruct(ctypes.Structure):
     """Mirror of ``ffn_mi355x_plan``."""
 
@@ -157,13 +161,23 @@ def check(rc: int) -> None:
     raise RuntimeError(msg)
 
 
+def memo(lib) -> dict:
+    """Values derived from a loaded library that never change while it is loaded (device
+    properties, tile descriptions, plans of a key), kept on the handle itself: a one-shot ffn()
+    otherwise spends more host time on them than the GPU spends on a decode layer."""
+    return lib.__dict__.setdefault("_ffn_memo", {})
+
+
 def query(device: int) -> tuple[int, str]:
     """(CU count, gcnArchName) of a device; RuntimeError unless it is gfx950."""
     lib = load()
-    cus = ctypes.c_int(0)
-    arch = ctypes.create_string_buffer(64)
-    check(lib.ffn_mi355x_query(device, ctypes.byref(cus), arch, len(arch)))
-    return cus.value, arch.value.decode()
+    known = memo(lib).get(("device", device))
+    if known is None:
+        cus = ctypes.c_int(0)
+        arch = ctypes.create_string_buffer(64)
+        check(lib.ffn_mi355x_query(device, ctypes.byref(cus), arch, len(arch)))
+        known = memo(lib)["device", device] = (cus.value, arch.value.decode())
+    return known
 
 
 def activation_code(activation="gelu", gelu="erf") -> int:
@@ -178,12 +192,20 @@ def activation_code(activation="gelu", gelu="erf") -> int:
 def make_plan(mp, kp, hp, np_, dtype, down_impl, gelu, block_num, up_variant=-1,
               down_variant=-1, m=None, activation="gelu") -> PlanStruct:
     """Native plan; `m` is the logical row count (default: all mp rows hold data); `gelu` is the
-    GELU form when activation is 'gelu'."""
+    GELU form when activation is 'gelu'.  A key planned before returns a copy of its plan (the
+    plan is a function of the arguments alone); at most MAX_PLANS are kept."""
+    lib = load()
+    args = (mp if m is None else m, mp, kp, hp, np_, dtype, DOWN_CODES[down_impl],
+            activation_code(activation, gelu), block_num, up_variant, down_variant)
+    plans = memo(lib).setdefault("plans", {})
+    known = plans.get(args)
+    if known is not None:
+        return PlanStruct.from_buffer_copy(known)
     plan = PlanStruct()
-    check(load().ffn_mi355x_make_plan(mp if m is None else m, mp, kp, hp, np_, dtype,
-                                      DOWN_CODES[down_impl],
-                                      activation_code(activation, gelu), block_num, up_variant,
-                                      down_variant, ctypes.byref(plan)))
+    check(lib.ffn_mi355x_make_plan(*args, ctypes.byref(plan)))
+    if len(plans) >= MAX_PLANS:
+        plans.clear()
+    plans[args] = bytes(plan)
     return plan
 
 
@@ -209,16 +231,22 @@ def set_x_rows(plan: PlanStruct, d1, d2, s0, s1, s2) -> None:
     check(load().ffn_mi355x_set_x_rows(ctypes.byref(plan), d1, d2, s0, s1, s2))
 
 
-def variants() -> list[dict]:
+def variant(v: int) -> dict:
+    """Geometry of one compiled tile variant."""
     lib = load()
-    out = []
-    for v in range(lib.ffn_mi355x_num_variants()):
+    known = memo(lib).get(("variant", v))
+    if known is None:
         vals = [ctypes.c_int(0) for _ in range(6)]
         check(lib.ffn_mi355x_variant_info(v, *map(ctypes.byref, vals)))
         refill = lib.ffn_mi355x_variant_refill_waves(v)
         check(min(refill, 0))
         edge = lib.ffn_mi355x_variant_mfma_edge(v)
         check(min(edge, 0))
-        out.append(dict(zip(("bm", "bn", "bk", "waves", "stages", "lds_bytes"),
-                            (x.value for x in vals)), variant=v, refill_waves=refill, mfma_edge=edge))
-    return out
+        known = memo(lib)["variant", v] = dict(
+            zip(("bm", "bn", "bk", "waves", "stages", "lds_bytes"), (x.value for x in vals)),
+            variant=v, refill_waves=refill, mfma_edge=edge)
+    return dict(known)
+
+
+def variants() -> list[dict]:
+    return [variant(v) for v in range(load().ffn_mi355x_num_variants())]

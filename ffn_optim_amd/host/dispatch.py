@@ -12,6 +12,8 @@ import ctypes
 import hashlib
 from dataclasses import dataclass
 
+from .. import _lib
+
 DOWN_IMPLS = ("basic", "full_load_a", "full_load_b", "streamk")
 GELU_FORMS = ("erf", "rational")
 # C-ABI entry point and the down-projection role it runs
@@ -54,25 +56,37 @@ class Selection:
         return self
 
 
+def _file_sha256(lib, path, stat):
+    """sha256 of the library file, read once per state of the file (device, inode, size, time):
+    hashing its 73 MB takes 45 ms, and every preparation asks for it."""
+    key = ("sha256", str(path), stat.st_dev, stat.st_ino, stat.st_size, stat.st_mtime_ns)
+    memo = _lib.memo(lib)
+    digest = memo.get(key)
+    if digest is None:
+        digest = memo[key] = hashlib.sha256(path.read_bytes()).hexdigest()
+    return digest
+
+
 def verify_dependency():
     """Check that the prebuilt gfx950 library is present and loadable; return its provenance."""
-    from .. import _lib
-
     path = _lib.LIBRARY_PATH
-    if not path.exists():
+    try:
+        stat = path.stat()
+    except OSError:
         raise DependencyUnavailable(
-            f"{path.name} is not built; run `python -m ffn_optim_amd.build` first")
+            f"{path.name} is not built; run `python -m ffn_optim_amd.build` first") from None
     try:
         lib = _lib.load()
     except OSError as exc:
         raise DependencyUnavailable(f"cannot load {path.name}: {exc}") from exc
     return {"library": str(path),
-            "library_sha256": hashlib.sha256(path.read_bytes()).hexdigest(),
+            "library_sha256": _file_sha256(lib, path, stat),
             "version": lib.ffn_mi355x_version().decode()}
 
 
-def compile_kernel(plan):
-    """Resolve the launch entry point for a plan; returns (artifact, provenance).
+def compile_kernel(plan, provenance=None):
+    """Resolve the launch entry point for a plan; returns (artifact, provenance).  `provenance` is
+    verify_dependency's result where the caller has just called it.
 
     The counterpart of the reference's compile step: the kernels are already
     compiled for gfx950, so this loads the library and binds the plan.  The
@@ -80,10 +94,8 @@ def compile_kernel(plan):
     the library lacks a launch entry point or the plan's tile variants (prepare_ffn
     reports it as KernelCompilationError).
     """
-    Selection(plan.selection.up_impl, plan.selection.down_impl).require_available()
-    provenance = verify_dependency()
-    from .. import _lib
-
+    plan.selection.require_available()
+    provenance = verify_dependency() if provenance is None else dict(provenance)
     lib = _lib.load()
     native = plan.native
     # binding: the entry points this artifact launches through, and the plan's tile variants

@@ -168,29 +168,51 @@ def operands_aligned(x, weight1, weight2, plan):
             and weight1.is_contiguous() and weight2.is_contiguous())
 
 
-def interleave_gate_up(weight, h, hp):
+def interleave_gate_up(weight, h, hp, width=None):
     """SwiGLU weight1 [2h, K] (gate rows, then up rows) or bias1 [2h] -> the [2hp, ...] layout the
     up GEMM reads: 32-row blocks alternate, block 2b holding gate rows 32b..32b+31 and block 2b+1
-    the up rows of the same hidden columns; zero past h."""
+    the up rows of the same hidden columns; zero past h, and past K when `width` is wider.  Every
+    element is written once."""
     import torch
     tail = tuple(weight.shape[1:])
-    out = torch.zeros((hp // 32, 2, 32) + tail, device=weight.device, dtype=weight.dtype)
-    flat = out.view((hp // 32, 2 * 32) + tail)
-    gate = torch.zeros((hp,) + tail, device=weight.device, dtype=weight.dtype)
-    up = torch.zeros_like(gate)
-    gate[:h].copy_(weight[:h])
-    up[:h].copy_(weight[h:2 * h])
-    out[:, 0].copy_(gate.view((hp // 32, 32) + tail))
-    out[:, 1].copy_(up.view((hp // 32, 32) + tail))
-    return flat.reshape((2 * hp,) + tail)
+    k = tail[0] if tail else 0
+    wide = (width,) if tail and width is not None else tail
+    out = torch.empty((hp // 32, 2, 32) + wide, device=weight.device, dtype=weight.dtype)
+    dst = out[..., :k] if wide != tail else out
+    blocks, rest = divmod(h, 32)
+    for half in range(2):
+        rows = weight[half * h:(half + 1) * h]
+        dst[:blocks, half].copy_(rows[:blocks * 32].unflatten(0, (blocks, 32)))
+        if rest:
+            dst[blocks, half, :rest].copy_(rows[blocks * 32:])
+    if rest:
+        out[blocks, :, rest:].zero_()
+    if hp // 32 > blocks + (rest > 0):
+        out[blocks + (rest > 0):].zero_()
+    if wide != tail:
+        out[..., k:].zero_()
+    return out.reshape((2 * hp,) + wide)
+
+
+def _padded(src, rows, cols, clean_rows):
+    """[rows, cols] buffer holding the 2-D src, zero past its columns; the rows past it are zeros
+    when clean_rows, else not written (the kernels' range checks never read them)."""
+    import torch
+    r, c = src.shape
+    out = torch.empty((rows, cols), device=src.device, dtype=src.dtype)
+    out[:r, :c].copy_(src)
+    if c < cols:
+        out[:, c:].zero_()
+    if clean_rows and r < rows:
+        out[r:].zero_()
+    return out
 
 
 def prepare_storage(x, weight1, weight2, plan, alias_aligned=False, bias1=None, bias2=None):
     """Contiguise and zero-pad into [mp,kp], [hp,kp], [np,hp]; allocate hidden, out, workspace.
 
     Same buffers as ops/host/inputs.py:74-90; the FP32 workspace holds the arrival counters and
-    partial tiles of the Stream-K down and of a split up GEMM (allocated zero-filled; every
-    partial slot is written before it is read).
+    partial tiles of a Stream-K or split Basic down and of a split up GEMM.
     Returns the six buffers, the operand layout (k, h, n, ldx, ldw1, ldw2) for
     ffn_mi355x_set_operands and X's row grid (d1, d2, s0, s1, s2) for ffn_mi355x_set_x_rows,
     or None when X is read as rows at pitch ldx.
@@ -207,9 +229,14 @@ def prepare_storage(x, weight1, weight2, plan, alias_aligned=False, bias1=None, 
     p = plan.problem
     hidden = torch.empty((plan.mp, plan.hp), device=x.device, dtype=x.dtype)
     out = torch.empty((plan.mp, plan.np), device=x.device, dtype=x.dtype)
-    # zero-filled: its leading bytes are the split tiles' arrival counters, which every launch
-    # leaves zero again
-    ws = torch.zeros(plan.workspace_shape, device=x.device, dtype=torch.float32)
+    ws = torch.empty(plan.workspace_shape, device=x.device, dtype=torch.float32)
+    # its leading bytes are the split tiles' arrival counters, which every launch leaves zero
+    # again (and a down's are cleared by the up launch before it); the partial slots are written
+    # before they are read
+    native = plan.native
+    if native.workspace_bytes and not (alias_aligned and native.up_sk_tiles == 0 and not native.single_launch):
+        from .. import _lib
+        ws.view(-1)[:_lib.workspace_counter_bytes(native) // 4].zero_()
     grid = row_grid(x, p.k) if alias_aligned else None
     x_rows = None
     if grid is not None and grid[0] == "pitch":
@@ -218,25 +245,20 @@ def prepare_storage(x, weight1, weight2, plan, alias_aligned=False, bias1=None, 
     elif grid is not None:
         xs, ldx, x_rows = x, p.k, grid[1]
     else:
-        xs = torch.zeros((plan.mp, plan.kp), device=x.device, dtype=x.dtype)
-        xs[:p.m, :p.k].copy_(x.reshape(p.m, p.k))
+        xs = _padded(x.reshape(p.m, p.k), plan.mp, plan.kp, not alias_aligned)
         ldx = plan.kp
     if p.activation == "swiglu":
         # always a copy: the gate and up rows are interleaved for the up GEMM
-        wk = torch.zeros((2 * p.h, plan.kp), device=x.device, dtype=x.dtype)
-        wk[:, :p.k].copy_(weight1)
-        w1s, ldw1 = interleave_gate_up(wk, p.h, plan.hp), plan.kp
+        w1s, ldw1 = interleave_gate_up(weight1, p.h, plan.hp, plan.kp), plan.kp
     elif alias_aligned and _in_place(weight1, p.k):
         w1s, ldw1 = weight1, p.k
     else:
-        w1s = torch.zeros((plan.hp, plan.kp), device=x.device, dtype=x.dtype)
-        w1s[:p.h, :p.k].copy_(weight1)
+        w1s = _padded(weight1, plan.hp, plan.kp, not alias_aligned)
         ldw1 = plan.kp
     if alias_aligned and _in_place(weight2, p.h):
         w2s, ldw2 = weight2, p.h
     else:
-        w2s = torch.zeros((plan.np, plan.hp), device=x.device, dtype=x.dtype)
-        w2s[:p.n, :p.h].copy_(weight2)
+        w2s = _padded(weight2, plan.np, plan.hp, not alias_aligned)
         ldw2 = plan.hp
     # the reduction runs to the logical K when both up operands hold whole chunks up to it
     k = p.k if p.k % 8 == 0 else plan.kp

@@ -9,7 +9,8 @@ from __future__ import annotations
 
 from dataclasses import asdict, dataclass
 
-from .dispatch import Selection
+from .. import _lib, tuning
+from .dispatch import GELU_FORMS, Selection
 from .inputs import Problem
 
 MI355X_CU_COUNT = 256
@@ -106,8 +107,7 @@ class Plan:
 
 
 def _tile(bm, bn, bk, variant):
-    from .. import _lib
-    info = _lib.variants()[variant]
+    info = _lib.variant(variant)
     return Tile(bm, bn, bk, info["waves"], info["stages"], variant)
 
 
@@ -121,9 +121,6 @@ def make_plan(problem, selection=Selection(), block_num=DEFAULT_BLOCK_NUM, *, ge
     and tuned=True, a measured choice from the tuning table (ffn_optim_amd.tuning)
     replaces the library planner's for the shapes it covers.
     """
-    from .. import _lib
-    from .dispatch import GELU_FORMS
-
     selection.require_available()
     if type(block_num) is not int or not 1 <= block_num <= 65535:
         raise ValueError("block_num must be a positive integer; hardware limit checked before launch")
@@ -134,7 +131,6 @@ def make_plan(problem, selection=Selection(), block_num=DEFAULT_BLOCK_NUM, *, ge
     dtype = _lib.BF16 if problem.dtype == "bfloat16" else _lib.FP16
     activation = getattr(problem, "activation", "gelu")
     if tuned and up_variant is None and down_variant is None:
-        from .. import tuning
         # the key's epilogue field: the GELU form, or the other activation's name
         epilogue = gelu if activation == "gelu" else activation
         hit = tuning.lookup(tuning.make_key(problem.m, mp, kp, hp, np_, problem.dtype,

@@ -13,6 +13,7 @@ A key is the padded problem plus everything that changes which kernels run:
 from __future__ import annotations
 
 import json
+import os
 import threading
 from pathlib import Path
 
@@ -41,9 +42,12 @@ def _key_tuple(key: dict) -> tuple:
 
 def load(path: Path | str | None = None) -> dict:
     """{key tuple: entry} of a table file; an absent file is an empty table."""
-    path = Path(path or TABLE_PATH)
+    path = TABLE_PATH if path is None else Path(path)
     with _lock:
-        mtime = path.stat().st_mtime if path.exists() else None
+        try:
+            mtime = os.stat(path).st_mtime
+        except OSError:
+            mtime = None
         cached = _cache.get(path)
         if cached is not None and cached["mtime"] == mtime:
             return cached["entries"]
