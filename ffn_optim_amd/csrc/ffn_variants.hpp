@@ -43,7 +43,12 @@
 // the memory-bound small-M (decode) shapes.  Variant 14 K-slices the 64x64 tile (64x32 wave
 // tiles over half of every stage): two MFMAs per k-step per wave instead of one, for the
 // latency-bound down GEMMs with one 64x64 tile per CU (-8 to -9% on the unaligned mid-size
-// and the decode Basic down).
+// and the decode Basic down).  Variant 16's four waves stand two along M (32x64 wave tiles over half
+// of every stage): each holds whole gate/up block pairs, so it is SwiGLU's narrow tile.  SwiGLU's other
+// tiles are 128 columns wide and leave a small-M up GEMM on half the CUs (against the best of
+// them, bf16, K -> H: 2 rows 4512 -> 7808 40.0 -> 27.6 us, 60 rows 4864 -> 6912 41.9 -> 31.1, 176 rows
+// 3296 -> 640 22.1 -> 14.6, 16 rows 2048 -> 5504 12.9 -> 10.4).  Variant 19, which GELU and the down
+// GEMM take, keeps two along N; an output's sum is the same either way.
 // Each variant is built for both storage types in its own object, with every launch role:
 // the up epilogues (GELU-erf, GELU-rational, SiLU, and SwiGLU where its wave tiles hold whole
 // 64-column block pairs), the plain store of the down GEMM, the Stream-K form of the store and
@@ -68,7 +73,7 @@
     X(13, 128, 128, 64, 2, 2, 4, 3, 2, 2)   \
     X(14, 64, 64, 64, 1, 2, 6, -1, 2, 2)    \
     X(15, 32, 32, 128, 1, 1, 8, -1, 4, 2)   \
-    X(16, 64, 64, 128, 1, 2, 5, -1, 4, 2)   \
+    X(16, 64, 64, 128, 2, 1, 5, -1, 4, 2)   \
     X(17, 256, 128, 64, 2, 2, 3, -1, 4, 1, 0, 4) \
     X(18, 128, 128, 64, 2, 2, 4, 3, 2, 2, 0, 4)  \
     X(19, 64, 64, 128, 1, 2, 5, -1, 4, 2, 0, 4)  \

@@ -142,6 +142,39 @@ def test_up_integer_activation_all_variants(dtype, activation):
     assert tested >= 8
 
 
+@pytest.mark.parametrize("m, k, h", [
+    (1, 200, 65), (63, 130, 576), (65, 1000, 640),
+    (16, 2048, 8192),   # 64 MiB of gate and up rows, 4 KiB pitch: tile columns rotate their K range
+])
+def test_swiglu_narrow_tile_edges(m, k, h):
+    """SwiGLU on the 64x64 tile (two waves along M, whole gate/up block pairs each) at the edges of
+    its tiles: one row, one short of a tile, one past it, ragged K and H.  Integer operands make z
+    exact: hidden is within one unit in the last place of the float64 SiLU(gate) * up."""
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(m)
+    mp, kp, hp = -(-m // 64) * 64, -(-k // 16) * 16, -(-h // 64) * 64
+    x, w1 = torch.zeros(mp, kp, dtype=torch.bfloat16), torch.zeros(2 * h, kp, dtype=torch.bfloat16)
+    x[:m, :k] = torch.randint(-2, 3, (m, k), generator=gen).bfloat16()
+    # 30 nonzero weights a row, anywhere in K: |z| <= 60 is exact, and e^60 keeps its FP32 reciprocal
+    # normal (past e^87.3 = 2^126 the kernels' SiLU flushes to zero, where float64's does not)
+    cols = torch.rand(2 * h, k, generator=gen).topk(30, dim=1).indices
+    w1.scatter_(1, cols, (torch.randint(0, 2, cols.shape, generator=gen) * 2 - 1).bfloat16())
+    z = (x.float() @ w1.float().T).double()
+    assert float(z.abs().max()) <= 60
+    truth = torch.zeros(mp, hp, dtype=torch.bfloat16)
+    truth[:, :h] = (z[:, :h] / (1 + torch.exp(-z[:, :h])) * z[:, h:]).bfloat16()
+    plan = _lib.make_plan(mp, kp, hp, 64, _lib.BF16, "basic", "erf", 256, 16, -1, m=m, activation="swiglu")
+    assert (plan.up_bm, plan.up_bn) == (64, 64)
+    hidden = torch.full((mp, hp), float("nan"), dtype=torch.bfloat16, device="cuda")
+    xd, w1d = x.cuda(), interleave_gate_up(w1, h, hp).contiguous().cuda()
+    _lib.check(lib.ffn_mi355x_up(ctypes.byref(plan), xd.data_ptr(), w1d.data_ptr(), hidden.data_ptr(), None,
+                                 torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    ulps = (_ordinal(hidden.cpu().view(torch.int16)) - _ordinal(truth.view(torch.int16))).abs()
+    say("swiglu-narrow", m, k, h, int(ulps.max()))
+    assert int(ulps.max()) <= 1
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_down_integer_bias_bit_exact(dtype):
     """Integer hidden, W2 and bias2: out = hidden W2^T + b2 is exact in FP32 and rounded once, for
