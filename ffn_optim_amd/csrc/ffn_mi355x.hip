@@ -301,14 +301,27 @@ bool split_whole(const Variant& v, long long m_valid, long long N, long long K, 
     return true;
 }
 
-// A Basic down splits its tiles the same way where the model prices that below whole tiles, and
-// the pieces cut a tile's iterations evenly.  Whole tiles left CUs idle on small-M FFNs, whose
-// output is few tiles wide: 128x4096 -> 16384 -> 4096, 128 tiles of 64x64 whole 71.3 us, split in
-// two 46.1, 64 of 64x128 split in four 45.2; 256 rows 71.3 -> 57.2; 512 rows 106.8 (64x128 whole) ->
-// 81.9 (256x128 split); 512x1024 -> 4096 -> 1024, 13.3 -> 11.2.
-bool split_down(const Variant& v, long long M, long long m_valid, long long N, long long K, int G, SkShape& s) {
-    return split_whole(v, m_valid, N, K, G, s) && s.k_iters % s.pieces == 0 &&
-           cost_streamk(v, s, m_valid, N, K) < cost_basic(v, M, m_valid, N, K, G);
+// A Basic down splits its tiles the same way where the model prices that below whole tiles.  Whole
+// tiles left CUs idle on small-M FFNs, whose output is few tiles wide: 128x4096 -> 16384 -> 4096,
+// 128 tiles of 64x64 whole 71.3 us, split in two 46.1, 64 of 64x128 split in four 45.2; 256 rows
+// 71.3 -> 57.2; 512 rows 106.8 (64x128 whole) -> 81.9 (256x128 split); 512x1024 -> 4096 -> 1024,
+// 13.3 -> 11.2.  Depths below kSplitDownMinK stay whole: the model prices a short tile's iterations
+// too high (the K-sliced 64x64 tile whole against split: 2048 deep 8.1 and 8.5 us; 2304 deep
+// 9.57 and 9.63, its FFN 41.8 and 42.5; 2752 deep 8.9 and 8.5; 3072 deep 11.2 and 9.1).
+// Pieces that do not cut a tile's iterations evenly run on from one tile into the next: two
+// partials and two finishes for most workgroups.  They are priced half as much again (32x32 tile
+// whole against split: 1 row, 6208 deep, 512 wide 13.0 and 11.1 us; 32 rows, 9088 deep, 3072 wide
+// 18.0 and 15.7; 64 rows, 5504 deep, 2048 wide 11.1 and 13.1, which stays whole).
+constexpr long long kSplitDownMinK = 2560;
+constexpr double kUnevenPieces = 1.5;
+bool split_down(const Variant& v, long long M, long long m_valid, long long N, long long K, int G, SkShape& s,
+                double& cost) {
+    cost = cost_basic(v, M, m_valid, N, K, G);
+    if (K < kSplitDownMinK || !split_whole(v, m_valid, N, K, G, s)) return false;
+    const double c = cost_streamk(v, s, m_valid, N, K) * (s.k_iters % s.pieces == 0 ? 1.0 : kUnevenPieces);
+    if (c >= cost) return false;
+    cost = c;
+    return true;
 }
 
 int pick_basic(long long M, long long m_valid, long long N, long long K, int G) {
@@ -316,9 +329,8 @@ int pick_basic(long long M, long long m_valid, long long N, long long K, int G) 
     double best_cost = 1e300;
     for (int i = 0; i < kNumVariants; ++i) {
         SkShape s;
-        const double c = split_down(kVariants[i], M, m_valid, N, K, G, s)
-                             ? cost_streamk(kVariants[i], s, m_valid, N, K)
-                             : cost_basic(kVariants[i], M, m_valid, N, K, G);
+        double c;
+        split_down(kVariants[i], M, m_valid, N, K, G, s, c);
         if (better(c, kVariants[i], best_cost, kVariants[best], m_valid)) best_cost = c, best = i;
     }
     return best;
@@ -647,7 +659,7 @@ int ffn_mi355x_make_plan(int m, int mp, int kp, int hp, int np, int dtype, int d
     // down: [mp x np], depth hp
     int dv;
     bool split_basic = false;
-    SkShape sb;
+    SkShape sb{};
     if (down_impl == FFN_MI355X_DOWN_STREAMK) {
         if (down_variant >= 0) {
             SkShape s;
@@ -677,7 +689,14 @@ int ffn_mi355x_make_plan(int m, int mp, int kp, int hp, int np, int dtype, int d
         }
     } else {
         dv = down_variant >= 0 ? down_variant : pick_basic(mp, m, np, hp, G);
-        split_basic = split_down(kVariants[dv], mp, m, np, hp, G, sb);
+        double price;
+        split_basic = split_down(kVariants[dv], mp, m, np, hp, G, sb, price);
+        // whole tiles where a large block_num's pieces outgrow the counters or the 32-bit slot
+        // offsets: a Basic plan is not refused for a split nobody asked for
+        const size_t words = (size_t)sb.sk * kVariants[dv].nw + (size_t)plan->up_sk_tiles * U.nw;
+        const size_t slots = (size_t)sb.grid * sb.slots * kVariants[dv].bm * kVariants[dv].bn * 4u;
+        if (split_basic && (words > kCounterBytes / 4 || slots + flags_bytes(plan) >= (size_t)1 << 31))
+            split_basic = false;
     }
     const Variant& D = kVariants[dv];
     plan->down_variant = dv;

@@ -117,3 +117,29 @@ def test_split_basic_in_place_operands_match_their_copies():
     first = prepared.run().clone()
     assert torch.equal(first, prepared.run())
     assert torch.equal(first, ffn(x, w1, w2))
+
+
+@pytest.mark.parametrize("m, h, n", [
+    (1, 6161, 512),     # 49 iterations in four pieces: all but the first straddle two tiles
+    (32, 9088, 3072),   # 71 iterations in two
+    (65, 2560, 192),    # the shallowest depth that splits, in even pieces
+    (65, 2496, 192),    # one step shallower: whole
+])
+def test_split_basic_down_by_depth(m, h, n):
+    """The automatic Basic down at the edges of its split: pieces that do not cut a tile evenly, and
+    the depth below which tiles stay whole; exact against the float product, run after run."""
+    lib = _lib.load()
+    hp, np_ = _align(h, 64), _align(n, 64)
+    hid, w2, golden = _operands(m, h, n, hp, np_, torch.bfloat16, h)
+    hid_d, w2_d = hid.cuda(), w2.cuda()
+    plan = _lib.make_plan(hid.shape[0], 64, hp, np_, _lib.BF16, "basic", "erf", 256, m=m)
+    assert (plan.down_sk_tiles > 0) == (h >= 2560)
+    ws = poisoned_workspace(plan)
+    say("depth", m, h, n, plan.down_variant, plan.down_tiles, plan.down_grid)
+    for _ in range(3):
+        out = torch.full(golden.shape, float("nan"), dtype=torch.bfloat16, device="cuda")
+        _lib.check(lib.ffn_mi355x_down(ctypes.byref(plan), hid_d.data_ptr(), w2_d.data_ptr(), out.data_ptr(),
+                                       ws.data_ptr(), torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        assert torch.equal(out.cpu()[:m].view(torch.int16), golden[:m].view(torch.int16))
+        assert counters_are_zero(plan, ws)

@@ -770,6 +770,34 @@ def test_basic_down_splits_only_where_whole_tiles_leave_workgroups_idle(m, k, h,
                                  + n.down_grid * n.down_slots_per_wg * n.down_bm * n.down_bn * 4)
 
 
+@pytest.mark.parametrize("m, k, h, n, grid", [
+    (1, 512, 6208, 512, 64),       # 49 iterations in four pieces (13.0 -> 11.1 us)
+    (32, 3072, 9088, 3072, 192),   # 71 in two (18.0 -> 15.7)
+    (64, 2048, 5504, 2048, 128),   # 43 in two would take 13.1 us, whole tiles 11.1
+    (416, 6864, 2304, 768, 84),    # too shallow to split
+])
+def test_basic_down_uneven_and_shallow_splits(m, k, h, n, grid):
+    """Pieces that do not cut a tile evenly straddle tiles and are taken only where they pay well;
+    shallow reductions stay whole.  Pieces hold all (tile, iteration) pairs: the grid covers them."""
+    p = problem_from_shapes((m, k), (h, k), (n, h), "bfloat16")
+    native = make_plan(p, Selection("basic", "basic"), 256, tuned=False).native
+    assert native.down_grid == grid
+    split = native.down_sk_tiles > 0
+    assert split == (grid > native.down_tiles)
+    if split:
+        span = -(-native.down_tiles * native.down_k_iters // native.down_grid)
+        assert native.down_slots_per_wg >= 2 >= -(-span // native.down_k_iters) + 1
+
+
+@pytest.mark.parametrize("block_num", [256, 4096, 65535])
+def test_large_block_num_never_refuses_a_basic_plan(block_num):
+    """A block_num whose split pieces would outgrow the counters or the slot offsets gets whole tiles."""
+    for m, k, h in ((4096, 1024, 8192), (8192, 3072, 12288), (128, 4096, 16384)):
+        for variant in (-1, 0, 5, 20):
+            p = _lib.make_plan(m, k, h, k, _lib.BF16, "basic", "erf", block_num, 3, variant)
+            assert p.workspace_bytes < 1 << 31
+
+
 def test_swiglu_up_takes_narrow_tiles_at_small_m():
     """SwiGLU up tiles at few rows: 64x64 where 128 columns leave CUs idle (12.9 -> 10.4 us), and
     64 rows rather than 128 of which half hold no data (44.6 -> 37.7 us)."""
