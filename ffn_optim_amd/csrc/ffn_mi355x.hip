@@ -135,7 +135,7 @@ double tile_eff(const Variant& v, bool up = false) {
     // FFN's Basic down: 512 tiles of it took 30.7 us against 27.0 us for 128 of 64x64, one tuning
     // run).  0.38 and 0.19 order the tiles of 32 FFN shapes timed in one run (16 to 4096 rows,
     // whole and split): the picks average 1% behind the fastest tile; at 0.3 and 0.15, 4%.
-    if (v.wgk > 1) return refill * (a >= 128 ? (v.nw + v.prod >= 8 ? 0.9 : 0.85) : a >= 64 ? 0.38 : 0.19);
+    if (v.wgk > 1) return refill * (a >= 128 ? (v.nw + v.prod >= 8 ? 0.9 : 0.85) : a >= 64 ? (v.nw + v.prod >= 8 ? 0.38 : 0.34) : 0.19);
     if (a >= 256) return refill * 1.0;
     // 256x192 (16x16 blocks): 0.92 per FLOP of the 256x256 tile, from the DiT-size up at eight
     // tiles per CU (493.5 against 453.0 us at six of 256x256) and its H/8 shard at one wave of
@@ -312,13 +312,24 @@ bool split_whole(const Variant& v, long long m_valid, long long N, long long K, 
 // partials and two finishes for most workgroups.  They are priced half as much again (32x32 tile
 // whole against split: 1 row, 6208 deep, 512 wide 13.0 and 11.1 us; 32 rows, 9088 deep, 3072 wide
 // 18.0 and 15.7; 64 rows, 5504 deep, 2048 wide 11.1 and 13.1, which stays whole).
+// Uneven pieces of more than two a tile are left out where they would take over half of the
+// workgroups (32 rows, 1536 -> 6210 -> 1536, 48 tiles in four: FFN 18.35 whole, 18.62 split), and so
+// are those of short tiles (3 rows, 768 -> 4685 -> 768, 37 iterations in four: 15.7 whole, 16.3 split).
 constexpr long long kSplitDownMinK = 2560;
 constexpr double kUnevenPieces = 1.5;
+constexpr long long kUnevenMinIters = 48;
+// Splits competing with whole tiles: near ties lost (64 rows, 1536 -> 5888 up: FFN 16.9 us whole, 17.9
+// split; 368 rows, 512 -> 3584 down: 17.0 and 17.3).
+constexpr double kSplitMargin = 1.1;
+double split_price(const Variant& v, const SkShape& s, long long m_valid, long long N, long long K, bool up = false) {
+    return cost_streamk(v, s, m_valid, N, K, up) * (s.k_iters % s.pieces == 0 ? kSplitMargin : kUnevenPieces);
+}
 bool split_down(const Variant& v, long long M, long long m_valid, long long N, long long K, int G, SkShape& s,
                 double& cost) {
     cost = cost_basic(v, M, m_valid, N, K, G);
     if (K < kSplitDownMinK || !split_whole(v, m_valid, N, K, G, s)) return false;
-    const double c = cost_streamk(v, s, m_valid, N, K) * (s.k_iters % s.pieces == 0 ? 1.0 : kUnevenPieces);
+    if (s.k_iters % s.pieces != 0 && (s.k_iters < kUnevenMinIters || (s.pieces > 2 && 2 * s.grid > G))) return false;
+    const double c = split_price(v, s, m_valid, N, K);
     if (c >= cost) return false;
     cost = c;
     return true;
@@ -366,6 +377,12 @@ bool swiglu_tile(const Variant& v) { return (v.bn / v.wgn) % 64 == 0; }
 // pieces priced ahead of 256 whole 64x128 tiles and measured 9-15% slower on the FFN; at 64 rows
 // and H 8192 only the 32x32 decode tiles fill the grid, and the split 64x64 tile stays 10%
 // ahead of them.
+//
+// Pieces that straddle tiles are priced as the down's (144 rows, 1070 -> 2304, 108 tiles of 64x64 in
+// two uneven pieces: FFN 22.5 us, whole 16.8).  SwiGLU's K-sliced 64x64 tile needs four iterations:
+// on fewer the exchange of its slices is not made up for (490 rows, 256 -> 592: FFN 12.2 us, on the
+// 64x128 tile 11.5; 112 rows, 512 deep: level; 1024 deep: 7.7 against 8.3).
+constexpr long long kSlicedSwigluMinK = 512;
 int pick_up(long long M, long long m_valid, long long N, long long K, int G, bool swiglu) {
     int best = -1;
     double best_cost = 1e300;
@@ -375,10 +392,11 @@ int pick_up(long long M, long long m_valid, long long N, long long K, int G, boo
                  cdiv(m_valid, kVariants[i].bm) * cdiv(N, kVariants[i].bn) * 2 > G;
     for (int i = 0; i < kNumVariants; ++i) {
         if (swiglu && !swiglu_tile(kVariants[i])) continue;
+        if (swiglu && kVariants[i].wgk > 1 && kVariants[i].bm < 128 && K < kSlicedSwigluMinK) continue;
         SkShape s;
         const bool split = !swiglu && split_whole(kVariants[i], m_valid, N, K, G, s);
         if (split && fills) continue;
-        const double c = split ? cost_streamk(kVariants[i], s, m_valid, N, K, true)
+        const double c = split ? split_price(kVariants[i], s, m_valid, N, K, true)
                                : cost_basic(kVariants[i], M, m_valid, N, K, G, true);
         if (best < 0 || better(c, kVariants[i], best_cost, kVariants[best], m_valid)) best_cost = c, best = i;
     }
