@@ -70,10 +70,12 @@ CORE_SIGNATURES = {
     "ffn_mi355x_strerror": (ctypes.c_char_p, [_i]),
     "ffn_mi355x_version": (ctypes.c_char_p, []),
 }
-# Launch entry points, bound when present: compile_kernel requires those a plan launches
+# Launch entry points (and the split of a plan's Basic down), bound when present: compile_kernel requires those a plan launches
 # through (require_entry_points), and a library without them fails there, the counterpart of
-# the reference's compile step failing (KernelCompilationError, ops/api.py:82-88).
+# the reference's compile step failing (KernelCompilationError, ops/api.py:82-88).  Without
+# ffn_mi355x_set_split_down every Basic down runs whole tiles.
 LAUNCH_SIGNATURES = {
+    "ffn_mi355x_set_split_down": (_i, [_P(PlanStruct), _i, _i]),
     "ffn_mi355x_run": (_i, [_P(PlanStruct), _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "ffn_mi355x_run_noalloc": (_i, [_P(PlanStruct), _vp, _vp, _vp, _vp, _vp, _vp]),
     "ffn_mi355x_run_ex": (_i, [_P(PlanStruct), _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
@@ -190,22 +192,27 @@ def activation_code(activation="gelu", gelu="erf") -> int:
 
 
 def make_plan(mp, kp, hp, np_, dtype, down_impl, gelu, block_num, up_variant=-1,
-              down_variant=-1, m=None, activation="gelu") -> PlanStruct:
+              down_variant=-1, m=None, activation="gelu", split_down=True) -> PlanStruct:
     """Native plan; `m` is the logical row count (default: all mp rows hold data); `gelu` is the
-    GELU form when activation is 'gelu'.  A key planned before returns a copy of its plan (the
-    plan is a function of the arguments alone); at most MAX_PLANS are kept."""
+    GELU form when activation is 'gelu'; split_down lets a Basic down split its tiles
+    (ffn_mi355x_set_split_down), for callers that allocate the plan's workspace_bytes.  A key
+    planned before returns a copy of its plan (the plan is a function of the arguments alone); at
+    most MAX_PLANS are kept."""
     lib = load()
     args = (mp if m is None else m, mp, kp, hp, np_, dtype, DOWN_CODES[down_impl],
             activation_code(activation, gelu), block_num, up_variant, down_variant)
+    split_down = bool(split_down) and DOWN_CODES[down_impl] == DOWN_CODES["basic"]
     plans = memo(lib).setdefault("plans", {})
-    known = plans.get(args)
+    known = plans.get((args, split_down))
     if known is not None:
         return PlanStruct.from_buffer_copy(known)
     plan = PlanStruct()
     check(lib.ffn_mi355x_make_plan(*args, ctypes.byref(plan)))
+    if split_down and "ffn_mi355x_set_split_down" not in lib._ffn_missing_launch:
+        check(lib.ffn_mi355x_set_split_down(ctypes.byref(plan), 1, down_variant))
     if len(plans) >= MAX_PLANS:
         plans.clear()
-    plans[args] = bytes(plan)
+    plans[args, split_down] = bytes(plan)
     return plan
 
 

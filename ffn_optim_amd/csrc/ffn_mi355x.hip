@@ -335,13 +335,15 @@ bool split_down(const Variant& v, long long M, long long m_valid, long long N, l
     return true;
 }
 
-int pick_basic(long long M, long long m_valid, long long N, long long K, int G) {
+// split: tiles are priced as split_down would run them, else whole.
+int pick_basic(long long M, long long m_valid, long long N, long long K, int G, bool split) {
     int best = 0;
     double best_cost = 1e300;
     for (int i = 0; i < kNumVariants; ++i) {
         SkShape s;
         double c;
-        split_down(kVariants[i], M, m_valid, N, K, G, s, c);
+        if (split) split_down(kVariants[i], M, m_valid, N, K, G, s, c);
+        else c = cost_basic(kVariants[i], M, m_valid, N, K, G);
         if (better(c, kVariants[i], best_cost, kVariants[best], m_valid)) best_cost = c, best = i;
     }
     return best;
@@ -520,9 +522,9 @@ unsigned long long plan_stamp(const ffn_mi355x_plan* p) {
     return h;
 }
 
-// A plan is used only as ffn_mi355x_make_plan (and ffn_mi355x_set_operands) left it: the grids,
-// tile counts, Stream-K split and workspace size it carries decide which memory the kernels
-// touch.  Both entry points derive them and stamp the plan; a plan whose fields no longer match
+// A plan is used only as ffn_mi355x_make_plan (and the ffn_mi355x_set_* calls) left it: the grids,
+// tile counts, splits and workspace size it carries decide which memory the kernels
+// touch.  The entry points derive them and stamp the plan; a plan whose fields no longer match
 // its stamp is refused.  (The stamp catches accidental edits of a plan, not forgery.)
 bool valid_plan(const ffn_mi355x_plan* p) {
     return p && p->stamp == plan_stamp(p) && p->m >= 1 && p->m <= p->mp && layout_ok(p) && p->up_variant >= 0 &&
@@ -533,13 +535,13 @@ bool valid_plan(const ffn_mi355x_plan* p) {
 }
 
 // Workspace layout: a fixed region of arrival counters first (one per split tile and wave, for
-// the split up GEMM and the Stream-K down alike, which run one after the other; every launch
+// the split up GEMM and a split down alike, which run one after the other; every launch
 // leaves them zero), then the FP32 partial-tile slots.  The region has the same size for every
 // plan, so one zero-filled workspace serves any plans in turn: no plan's slots overlap another
 // plan's counters.
 size_t flags_bytes(const ffn_mi355x_plan*) { return kCounterBytes; }
 
-// Arrival counters (one word per split tile and wave): the Stream-K down's from the start of the
+// Arrival counters (one word per split tile and wave): a split down's from the start of the
 // counter region, a split up GEMM's from its end, so that each GEMM's launch can clear the
 // other's (GemmParams::clear_words) without touching its own.
 // Each split tile's counters take a 128-byte line of their own (FFN_MI355X_SPLIT_COUNTER_WORDS
@@ -590,6 +592,90 @@ bool fused_ok(const ffn_mi355x_plan* p) {
            (p->activation == FFN_MI355X_GELU_ERF || p->activation == FFN_MI355X_GELU_RATIONAL) &&
            U.nw + U.prod == D.nw + D.prod && U.bm % D.bm == 0 && rbs >= 8 &&
            ffn::kFusedReady + rbs * ffn::kFusedStride <= (long long)(kCounterBytes / 4) && fast_dma_for(p->kp);
+}
+
+// Down GEMM of a plan whose up GEMM is planned, [mp x np], depth hp: its tile, its schedule and the
+// workspace of the two.  split: a Basic down may split its tiles (ffn_mi355x_set_split_down).
+int plan_down(ffn_mi355x_plan* plan, int down_variant, bool split) {
+    const int m = plan->m, mp = plan->mp, hp = plan->hp, np = plan->np, down_impl = plan->down_impl;
+    const int G = plan->block_num;
+    int dv;
+    bool split_basic = false;
+    SkShape sb{};
+    if (down_impl == FFN_MI355X_DOWN_STREAMK) {
+        if (down_variant >= 0) {
+            SkShape s;
+            if (!sk_shape(kVariants[down_variant], m, np, hp, G, s)) {
+                if (s.k_iters < 2)
+                    return fail(FFN_MI355X_ENOT_APPLICABLE,
+                                "Stream-K candidate requires at least two K tiles along H");
+                if (s.sk > 0)
+                    return fail(FFN_MI355X_ENOT_APPLICABLE,
+                                "Stream-K candidate splits more tiles (%lld) than the workspace counters "
+                                "hold for this block_num", s.sk);
+                return fail(FFN_MI355X_ENOT_APPLICABLE,
+                            "Stream-K candidate has no remainder tiles for this block_num");
+            }
+            dv = down_variant;
+        } else {
+            dv = pick_streamk(mp, m, np, hp, G);
+            if (dv < 0) {
+                bool any_two = false;
+                for (int i = 0; i < kNumVariants; ++i) any_two |= cdiv(hp, kVariants[i].bk) >= 2;
+                if (!any_two)
+                    return fail(FFN_MI355X_ENOT_APPLICABLE,
+                                "Stream-K candidate requires at least two K tiles along H");
+                return fail(FFN_MI355X_ENOT_APPLICABLE,
+                            "Stream-K candidate has no remainder tiles for this block_num");
+            }
+        }
+    } else {
+        dv = down_variant >= 0 ? down_variant : pick_basic(mp, m, np, hp, G, split);
+        double price;
+        split_basic = split && split_down(kVariants[dv], mp, m, np, hp, G, sb, price);
+        // whole tiles where a large block_num's pieces outgrow the counters or the 32-bit slot
+        // offsets
+        const size_t words = (size_t)sb.sk * kVariants[dv].nw +
+                             (size_t)plan->up_sk_tiles * kVariants[plan->up_variant].nw;
+        const size_t slots = (size_t)sb.grid * sb.slots * kVariants[dv].bm * kVariants[dv].bn * 4u;
+        if (split_basic && (words > kCounterBytes / 4 || slots + flags_bytes(plan) >= (size_t)1 << 31))
+            split_basic = false;
+    }
+    const Variant& D = kVariants[dv];
+    plan->down_variant = dv;
+    plan->down_bm = D.bm, plan->down_bn = D.bn, plan->down_bk = D.bk;
+    plan->down_tiles = (int)(cdiv(m, D.bm) * cdiv(np, D.bn));
+    plan->down_k_iters = (int)cdiv(hp, D.bk);
+    if (down_impl == FFN_MI355X_DOWN_STREAMK || split_basic) {
+        SkShape s = sb;
+        if (!split_basic) sk_shape(D, m, np, hp, G, s);
+        plan->down_dp_tiles = (int)s.dp;
+        plan->down_sk_tiles = (int)s.sk;
+        plan->down_slots_per_wg = (int)s.slots;
+        plan->down_grid = (int)s.grid;
+        plan->workspace_bytes = (size_t)s.grid * (size_t)s.slots * (size_t)D.bm * (size_t)D.bn * 4u;
+    } else {
+        plan->down_dp_tiles = plan->down_tiles;
+        plan->down_sk_tiles = plan->down_slots_per_wg = 0;
+        plan->down_grid = plan->down_tiles < G ? plan->down_tiles : G;
+        plan->workspace_bytes = 0;
+    }
+    plan->workspace_bytes = std::max(plan->workspace_bytes, up_partial_bytes(plan));
+    if (plan->workspace_bytes > 0) plan->workspace_bytes += flags_bytes(plan);
+    // The single launch is opt-in (ffn_mi355x_set_single_launch): measured against the two launches
+    // of the same tile pair it was slower on every workload it serves (aligned mid-size 78.6
+    // against 72.0 us, unaligned 45.4 against 30.2, DiT-size 1065 against 979).  A plan that can
+    // take it reserves the counter region, so its workspace serves either form.
+    plan->single_launch = 0;
+    if (fused_ok(plan) && plan->workspace_bytes < flags_bytes(plan)) plan->workspace_bytes = flags_bytes(plan);
+    if (up_counter_words(plan) + down_counter_words(plan) > kCounterBytes / 4)
+        return fail(FFN_MI355X_ENOT_APPLICABLE, "the split tiles of the two GEMMs need more arrival counters "
+                    "(%zu) than the workspace holds (%zu)", up_counter_words(plan) + down_counter_words(plan),
+                    kCounterBytes / 4);
+    // the kernels address partial slots with 32-bit buffer offsets
+    if (plan->workspace_bytes >= (size_t)1 << 31)
+        return fail(FFN_MI355X_EINVAL, "workspace of %zu bytes exceeds 2 GiB", plan->workspace_bytes);
+    return ok();
 }
 
 int launch(const Variant& v, int dtype, int role, const ffn::GemmParams& gp, int grid,
@@ -665,90 +751,15 @@ int ffn_mi355x_make_plan(int m, int mp, int kp, int hp, int np, int dtype, int d
     plan->up_tiles = (int)(cdiv(m, U.bm) * cdiv(un, U.bn));
     plan->up_grid = plan->up_tiles < G ? plan->up_tiles : G;
     plan->up_k_iters = (int)cdiv(kp, U.bk);
-    size_t up_ws = 0;
     SkShape su;
     if (!swiglu && split_whole(U, m, hp, kp, G, su)) {
         plan->up_sk_tiles = (int)su.sk;
         plan->up_slots_per_wg = (int)su.slots;
         plan->up_grid = (int)su.grid;
-        up_ws = (size_t)su.grid * (size_t)su.slots * (size_t)U.bm * (size_t)U.bn * 4u;
     }
 
-    // down: [mp x np], depth hp
-    int dv;
-    bool split_basic = false;
-    SkShape sb{};
-    if (down_impl == FFN_MI355X_DOWN_STREAMK) {
-        if (down_variant >= 0) {
-            SkShape s;
-            if (!sk_shape(kVariants[down_variant], m, np, hp, G, s)) {
-                if (s.k_iters < 2)
-                    return fail(FFN_MI355X_ENOT_APPLICABLE,
-                                "Stream-K candidate requires at least two K tiles along H");
-                if (s.sk > 0)
-                    return fail(FFN_MI355X_ENOT_APPLICABLE,
-                                "Stream-K candidate splits more tiles (%lld) than the workspace counters "
-                                "hold for this block_num", s.sk);
-                return fail(FFN_MI355X_ENOT_APPLICABLE,
-                            "Stream-K candidate has no remainder tiles for this block_num");
-            }
-            dv = down_variant;
-        } else {
-            dv = pick_streamk(mp, m, np, hp, G);
-            if (dv < 0) {
-                bool any_two = false;
-                for (int i = 0; i < kNumVariants; ++i) any_two |= cdiv(hp, kVariants[i].bk) >= 2;
-                if (!any_two)
-                    return fail(FFN_MI355X_ENOT_APPLICABLE,
-                                "Stream-K candidate requires at least two K tiles along H");
-                return fail(FFN_MI355X_ENOT_APPLICABLE,
-                            "Stream-K candidate has no remainder tiles for this block_num");
-            }
-        }
-    } else {
-        dv = down_variant >= 0 ? down_variant : pick_basic(mp, m, np, hp, G);
-        double price;
-        split_basic = split_down(kVariants[dv], mp, m, np, hp, G, sb, price);
-        // whole tiles where a large block_num's pieces outgrow the counters or the 32-bit slot
-        // offsets: a Basic plan is not refused for a split nobody asked for
-        const size_t words = (size_t)sb.sk * kVariants[dv].nw + (size_t)plan->up_sk_tiles * U.nw;
-        const size_t slots = (size_t)sb.grid * sb.slots * kVariants[dv].bm * kVariants[dv].bn * 4u;
-        if (split_basic && (words > kCounterBytes / 4 || slots + flags_bytes(plan) >= (size_t)1 << 31))
-            split_basic = false;
-    }
-    const Variant& D = kVariants[dv];
-    plan->down_variant = dv;
-    plan->down_bm = D.bm, plan->down_bn = D.bn, plan->down_bk = D.bk;
-    plan->down_tiles = (int)(cdiv(m, D.bm) * cdiv(np, D.bn));
-    plan->down_k_iters = (int)cdiv(hp, D.bk);
-    if (down_impl == FFN_MI355X_DOWN_STREAMK || split_basic) {
-        SkShape s = sb;
-        if (!split_basic) sk_shape(D, m, np, hp, G, s);
-        plan->down_dp_tiles = (int)s.dp;
-        plan->down_sk_tiles = (int)s.sk;
-        plan->down_slots_per_wg = (int)s.slots;
-        plan->down_grid = (int)s.grid;
-        plan->workspace_bytes = (size_t)s.grid * (size_t)s.slots * (size_t)D.bm * (size_t)D.bn * 4u;
-    } else {
-        plan->down_dp_tiles = plan->down_tiles;
-        plan->down_grid = plan->down_tiles < G ? plan->down_tiles : G;
-        plan->workspace_bytes = 0;
-    }
-    if (up_ws > plan->workspace_bytes) plan->workspace_bytes = up_ws;
-    if (plan->workspace_bytes > 0) plan->workspace_bytes += flags_bytes(plan);
-    // The single launch is opt-in (ffn_mi355x_set_single_launch): measured against the two launches
-    // of the same tile pair it was slower on every workload it serves (aligned mid-size 78.6
-    // against 72.0 us, unaligned 45.4 against 30.2, DiT-size 1065 against 979).  A plan that can
-    // take it reserves the counter region, so its workspace serves either form.
-    plan->single_launch = 0;
-    if (fused_ok(plan) && plan->workspace_bytes < flags_bytes(plan)) plan->workspace_bytes = flags_bytes(plan);
-    if (up_counter_words(plan) + down_counter_words(plan) > kCounterBytes / 4)
-        return fail(FFN_MI355X_ENOT_APPLICABLE, "the split tiles of the two GEMMs need more arrival counters "
-                    "(%zu) than the workspace holds (%zu)", up_counter_words(plan) + down_counter_words(plan),
-                    kCounterBytes / 4);
-    // the kernels address partial slots with 32-bit buffer offsets
-    if (plan->workspace_bytes >= (size_t)1 << 31)
-        return fail(FFN_MI355X_EINVAL, "workspace of %zu bytes exceeds 2 GiB", plan->workspace_bytes);
+    const int rc = plan_down(plan, down_variant, false);
+    if (rc != FFN_MI355X_OK) return rc;
     plan->k = kp, plan->h = hp, plan->n = np;
     plan->ldx = kp, plan->ldw1 = kp, plan->ldw2 = hp;
     plan->x_d1 = plan->x_d2 = plan->x_s0 = plan->x_s1 = plan->x_s2 = 0;
@@ -804,6 +815,23 @@ int ffn_mi355x_set_single_launch(ffn_mi355x_plan* plan, int on) {
     return ok();
 }
 
+int ffn_mi355x_set_split_down(ffn_mi355x_plan* plan, int on, int down_variant) {
+    if (!plan) return fail(FFN_MI355X_EINVAL, "plan must not be NULL");
+    if (!valid_plan(plan)) return fail(FFN_MI355X_EINVAL, "invalid plan");
+    if (down_variant >= kNumVariants)
+        return fail(FFN_MI355X_EINVAL, "tile variant out of range (0..%d)", kNumVariants - 1);
+    if (plan->down_impl != FFN_MI355X_DOWN_BASIC)
+        return fail(FFN_MI355X_ENOT_APPLICABLE, "a Stream-K down always splits its tiles");
+    if (plan->single_launch)
+        return fail(FFN_MI355X_ENOT_APPLICABLE, "the single launch runs whole down tiles");
+    ffn_mi355x_plan t = *plan;
+    const int rc = plan_down(&t, down_variant, on != 0);
+    if (rc != FFN_MI355X_OK) return rc;
+    t.stamp = plan_stamp(&t);
+    *plan = t;
+    return ok();
+}
+
 int ffn_mi355x_workspace_bytes(const ffn_mi355x_plan* plan, size_t* bytes) {
     if (!plan || !bytes) return fail(FFN_MI355X_EINVAL, "NULL argument");
     *bytes = plan->workspace_bytes;
@@ -829,19 +857,20 @@ void set_workspace(ffn::GemmParams& gp, const ffn_mi355x_plan* plan, void* ws, b
     gp.ws_bytes = (unsigned)(plan->workspace_bytes - f);
 }
 
-// Whether a call splits its plan's down GEMM.  A Basic down does so only in a workspace that holds
-// the plan's bytes: with none, a buffer that is too short (Basic plans have not always used one) or
-// the library's scratch it runs whole tiles.
+// Whether a call splits its plan's down GEMM.  A Basic down does so only where the plan was asked to
+// (ffn_mi355x_set_split_down), in a workspace of the caller's; with none, or in the library's
+// scratch, it runs whole tiles.  The bytes behind `ws` decide nothing: all that can be seen of them
+// is the HIP allocation around it, of which a pool's block is a part.
 bool down_is_split(const ffn_mi355x_plan* p, const void* ws, bool ws_scratch) {
     if (p->down_impl == FFN_MI355X_DOWN_STREAMK) return true;
-    return p->down_sk_tiles > 0 && ws && !ws_scratch && in_allocation(ws, p->workspace_bytes);
+    return p->down_sk_tiles > 0 && ws && !ws_scratch;
 }
 
-// Up GEMM of a plan.  ws_scratch: ws is this library's scratch array (its size is known, and it
-// is not a HIP allocation of its own to look up).
 // Rows of W1 a plan reads: the logical H, or for SwiGLU the 2 hp interleaved gate and up rows.
 long long w1_rows(const ffn_mi355x_plan* p) { return p->activation == FFN_MI355X_SWIGLU ? 2LL * p->hp : p->h; }
 
+// Up GEMM of a plan.  ws_scratch: ws is this library's scratch array (its size is known, and it
+// is not a HIP allocation of its own to look up).
 // built: fill *built and *role_out with the launch of an unsplit up GEMM instead of launching it.
 int run_up(const ffn_mi355x_plan* plan, const void* x, const void* w1, const void* b1, void* hidden, void* ws,
            bool ws_scratch, void* hip_stream, ffn::GemmParams* built = nullptr, int* role_out = nullptr) {

@@ -69,13 +69,13 @@ typedef struct ffn_mi355x_plan {
     int down_bm, down_bn, down_bk; /* down-projection macro tile (M x N x H) */
     int up_tiles, up_grid;
     int down_tiles, down_grid;   /* down_grid <= block_num: fewer for Basic when there are fewer
-                                    tiles, and for Stream-K or a split Basic down when that cuts
-                                    every split tile into equal pieces */
+                                    tiles, and where every tile is split (Stream-K or a split Basic
+                                    down): down_tiles times the pieces a tile, which are equal when
+                                    they divide down_k_iters and straddle two tiles otherwise */
     int down_k_iters;            /* BK-deep iterations along H per down tile */
     int down_dp_tiles;           /* tiles reduced whole by one workgroup */
-    int down_sk_tiles;           /* tiles whose H-range is split over workgroups; a Basic down splits
-                                    all of its tiles or none (whole tiles would leave at least half
-                                    of block_num idle: a small M) */
+    int down_sk_tiles;           /* tiles whose H-range is split over workgroups; 0 for a Basic down
+                                    unless ffn_mi355x_set_split_down split it (all of its tiles) */
     int down_slots_per_wg;       /* FP32 partial-tile slots per workgroup */
     size_t workspace_bytes;      /* FP32 partial-tile slots of a split down and the split up */
     /* Operand layout.  ffn_mi355x_make_plan sets the padded buffers (k = kp, h = hp,
@@ -100,8 +100,8 @@ typedef struct ffn_mi355x_plan {
        0, the two launches having measured faster); 0: two stream-ordered launches, up then
        down. */
     int single_launch;
-    /* Check word over every field above, written by ffn_mi355x_make_plan and
-       ffn_mi355x_set_operands.  The run entry points refuse a plan whose fields no longer
+    /* Check word over every field above, written by ffn_mi355x_make_plan and the
+       ffn_mi355x_set_* calls.  The run entry points refuse a plan whose fields no longer
        match it (EINVAL "invalid plan"): its grids, tile counts and workspace size decide
        which memory the kernels touch, so a plan is used only as the library left it. */
     unsigned long long stamp;
@@ -155,21 +155,32 @@ int ffn_mi355x_set_x_rows(ffn_mi355x_plan* plan, int d1, int d2, int s0, int s1,
  * reference, whose FFN is always one artifact (ops/api.py:43). */
 int ffn_mi355x_set_single_launch(ffn_mi355x_plan* plan, int on);
 
+/* Lets a Basic plan split its down GEMM's tiles along H over several workgroups (on = 1), as the
+ * Stream-K down and the split up do, where whole tiles would leave at least half of block_num
+ * idle (a small M) and the split is expected to be faster; 0 goes back to whole tiles, as
+ * ffn_mi355x_make_plan plans them.  The down's tile is chosen anew: down_variant as for
+ * ffn_mi355x_make_plan.  down_sk_tiles says whether the plan splits, and workspace_bytes grows when it
+ * does, so a caller turns this on only if it allocates workspace_bytes afterwards.  Operand
+ * layout and row grid are kept.  ENOT_APPLICABLE for a Stream-K plan and for one set to the
+ * single launch, which runs whole tiles; the plan is unchanged on failure.  No counterpart in the
+ * reference, whose Basic down never splits (ops/kernel/ffn.py:377-529). */
+int ffn_mi355x_set_split_down(ffn_mi355x_plan* plan, int on, int down_variant);
+
 /* Workspace bytes a plan uses (0 for a Basic down of whole tiles without a split up GEMM or a
  * single launch).  A plan whose only use of it is a split Basic down also runs without: see
  * ffn_mi355x_run. */
 int ffn_mi355x_workspace_bytes(const ffn_mi355x_plan* plan, size_t* bytes);
 
 /* Bytes at the start of every workspace that hold the split tiles' arrival counters (one
- * 32-bit counter per split tile and wave: the Stream-K down's from the start of the region, a
- * split up GEMM's from its end; each split tile's counters start FFN_MI355X_SPLIT_COUNTER_WORDS
+ * 32-bit counter per split tile and wave: a split down's, Stream-K or Basic, from the start of the
+ * region, a split up GEMM's from its end; each split tile's counters start FFN_MI355X_SPLIT_COUNTER_WORDS
  * words after the previous tile's when both GEMMs' split tiles fit the region that way, else
- * they are packed, one word per wave of the tile).  Each GEMM's launch clears the other's counters before any
- * tile, and every launch leaves its own zero: a Stream-K down therefore always starts from zero
- * counters when its up GEMM ran first in the same call (ffn_mi355x_run, or ffn_mi355x_up given
- * the workspace), whatever the region held, and a split up GEMM from its second call on.  Zero
- * the region before the first call of a plan with a split up GEMM (e.g. allocate the workspace
- * zero-filled).  A workspace can then serve any plans whose workspace_bytes it covers, one call
+ * they are packed, one word per wave of the tile).  Each GEMM's launch clears the other's
+ * counters before any tile, and every launch leaves its own zero: a split down therefore always
+ * starts from zero counters when its up GEMM ran first in the same call (ffn_mi355x_run, or
+ * ffn_mi355x_up given the workspace), whatever the region held, and a split up GEMM from its
+ * second call on.  Zero the region before the first call of a plan with a split up GEMM, and
+ * before a split down that runs without its up GEMM (e.g. allocate the workspace zero-filled).  A workspace can then serve any plans whose workspace_bytes it covers, one call
  * after another; calls that overlap on one workspace race.  The rest of the workspace needs no
  * initialisation.  No counterpart in the reference, whose Stream-K reduction is a separate
  * phase (ops/kernel/ffn.py:1035-1175). */
@@ -185,9 +196,11 @@ int ffn_mi355x_workspace_counter_bytes(const ffn_mi355x_plan* plan, size_t* byte
  * the single artifact(*tensors, block_num) launch of ops/api.py:43 built by
  * compile_kernel (ops/host/dispatch.py:97-116) from ops/kernel/ffn.py.
  * `ws` must hold plan->workspace_bytes for a Stream-K down or a split up, its counter bytes as
- * FFN_MI355X_WORKSPACE_COUNTER_BYTES describes.  A Basic down splits its tiles (down_sk_tiles)
- * only when it is given those bytes, and runs whole tiles when `ws` is NULL or shorter (the same
- * sums in another order); without a split GEMM `ws` may be NULL too.
+ * FFN_MI355X_WORKSPACE_COUNTER_BYTES describes; without a split GEMM it is not used and may be NULL.
+ * A plan whose Basic down was split (ffn_mi355x_set_split_down) takes a `ws` of
+ * plan->workspace_bytes, or NULL unless its up GEMM is split too: it then runs whole tiles of the
+ * planned size (the same sums in another order).  A `ws` that visibly ends earlier, at the end of
+ * its HIP allocation, is refused with FFN_MI355X_EINVAL; the end of a pool's block cannot be seen.
  * The Stream-K down is one launch: the pieces of a split tile store FP32 partial tiles to `ws`,
  * and the last piece to arrive sums them in ascending K order, rounds once and stores the tile.
  * A split up is the same with the GELU applied after the sum. */
@@ -201,13 +214,14 @@ int ffn_mi355x_run(const ffn_mi355x_plan* plan, const void* x, const void* w1,
  * tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.
  * The Stream-K partial tiles (and those of a split up GEMM) go to a scratch array of the
  * library itself, FFN_MI355X_NOALLOC_SCRATCH_BYTES per GPU; the caller passes the operands,
- * hidden and out as for ffn_mi355x_run, and no workspace.  A plan whose workspace_bytes exceeds
- * the scratch is refused with FFN_MI355X_EINVAL before any launch.  The call allocates and
+ * hidden and out as for ffn_mi355x_run, and no workspace.  A plan that needs more than the
+ * scratch is refused with FFN_MI355X_EINVAL before any launch (its workspace_bytes; a Basic down
+ * runs whole tiles here, so the bytes of its split do not count).  The call allocates and
  * frees nothing.  Every call on one GPU shares that GPU's scratch: calls that overlap on one GPU
  * (on different streams, or from different threads) race and must be serialised by the caller.
  * The scratch starts zero-filled and every call leaves its arrival counters zero again; every
- * partial is written before it is read within a call, so nothing needs clearing.  A Basic down
- * runs whole tiles here, so a Basic plan without a split up GEMM shares nothing between calls. */
+ * partial is written before it is read within a call, so nothing needs clearing.  A Basic plan
+ * without a split up GEMM or a single launch uses no scratch and shares nothing between calls. */
 int ffn_mi355x_run_noalloc(const ffn_mi355x_plan* plan, const void* x, const void* w1,
                            const void* w2, void* hidden, void* out, void* hip_stream);
 

@@ -620,7 +620,7 @@ def test_dirty_counter_region_is_repaired(fill):
         info = _lib.variants()
         words = ws[:_lib.workspace_counter_bytes(plan) // 4].view(torch.int32)
         tile_waves = lambda v: info[v]["waves"] - info[v]["refill_waves"]
-        down_sk = plan.down_sk_tiles if plan.down_impl == 1 else 0
+        down_sk = plan.down_sk_tiles    # Stream-K or split Basic
         spread = (down_sk + plan.up_sk_tiles) * _lib.SPLIT_COUNTER_WORDS <= words.numel()
         stride = lambda v: _lib.SPLIT_COUNTER_WORDS if spread else tile_waves(v)
         down = down_sk * stride(plan.down_variant)

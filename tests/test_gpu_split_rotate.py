@@ -143,3 +143,106 @@ def test_split_basic_down_by_depth(m, h, n):
         torch.cuda.synchronize()
         assert torch.equal(out.cpu()[:m].view(torch.int16), golden[:m].view(torch.int16))
         assert counters_are_zero(plan, ws)
+
+
+GUARD = 0x5A5A5A5A
+
+
+def _ffn_operands(m, k, h, n, plan):
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    mp, kp, hp, np_ = plan.mp, plan.kp, plan.hp, plan.np
+    x = torch.zeros((mp, kp), dtype=torch.bfloat16, device="cuda")
+    w1 = torch.zeros((hp, kp), dtype=torch.bfloat16, device="cuda")
+    w2 = torch.zeros((np_, hp), dtype=torch.bfloat16, device="cuda")
+    for t, rows, cols, std in ((x, m, k, 1.0), (w1, h, k, k ** -0.5), (w2, n, h, h ** -0.5)):
+        t[:rows, :cols] = (torch.randn((rows, cols), generator=gen, device="cuda") * std).bfloat16()
+    hidden = torch.empty((mp, hp), dtype=torch.bfloat16, device="cuda")
+    return x, w1, w2, hidden
+
+
+def _run_ffn(plan, x, w1, w2, hidden, ws_ptr):
+    out = torch.full((plan.mp, plan.np), float("nan"), dtype=torch.bfloat16, device="cuda")
+    hidden.fill_(float("nan"))
+    _lib.check(_lib.load().ffn_mi355x_run(ctypes.byref(plan), x.data_ptr(), w1.data_ptr(), w2.data_ptr(),
+                                          hidden.data_ptr(), out.data_ptr(), ws_ptr,
+                                          torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    return out
+
+
+def _plain_plan(m, k, h, n):
+    return _lib.make_plan(_align(m, 64), _align(k, 16), _align(h, 64), _align(n, 64), _lib.BF16, "basic", "erf", 256,
+                          m=m, split_down=False)
+
+
+@pytest.mark.parametrize("m, k, h, n", [(8, 6784, 11648, 320), (3, 4832, 7232, 640), (128, 4096, 16384, 4096)])
+def test_plain_basic_plan_leaves_ws_alone(m, k, h, n):
+    """A Basic plan nobody asked to split ignores `ws`: a 64-byte block of a larger buffer, a block whose
+    words are no counters, and NULL give the same bits, and the buffer keeps every word."""
+    plan = _plain_plan(m, k, h, n)
+    assert plan.workspace_bytes == 0 and plan.down_sk_tiles == 0
+    x, w1, w2, hidden = _ffn_operands(m, k, h, n, plan)
+    say("plain", m, k, h, n)
+    expected = _run_ffn(plan, x, w1, w2, hidden, None)
+    pool = torch.full((32 << 20,), GUARD, dtype=torch.int32, device="cuda")   # room for any split of these shapes
+    got = _run_ffn(plan, x, w1, w2, hidden, pool.data_ptr())
+    assert torch.equal(got, expected) and bool((pool == GUARD).all())
+    # the two stages on their own, the up without a workspace
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    out = torch.full_like(expected, float("nan"))
+    _lib.check(lib.ffn_mi355x_up(ctypes.byref(plan), x.data_ptr(), w1.data_ptr(), hidden.data_ptr(), None, stream))
+    _lib.check(lib.ffn_mi355x_down(ctypes.byref(plan), hidden.data_ptr(), w2.data_ptr(), out.data_ptr(),
+                                   pool.data_ptr(), stream))
+    torch.cuda.synchronize()
+    assert torch.equal(out, expected) and bool((pool == GUARD).all())
+
+
+def test_plain_basic_plan_with_split_up_takes_the_ups_workspace():
+    """A plain Basic plan with a split up GEMM needs the up's bytes alone, and stays inside them."""
+    m, k, h, n = 3, 7552, 3328, 3712
+    plan = _plain_plan(m, k, h, n)
+    assert plan.up_sk_tiles > 0 and plan.down_sk_tiles == 0
+    x, w1, w2, hidden = _ffn_operands(m, k, h, n, plan)
+    clean = poisoned_workspace(plan)
+    expected = _run_ffn(plan, x, w1, w2, hidden, clean.data_ptr())
+    pool = torch.full((32 << 20,), GUARD, dtype=torch.int32, device="cuda")
+    words = plan.workspace_bytes // 4
+    pool[:words] = poisoned_workspace(plan).view(torch.int32)
+    say("up-sized", plan.workspace_bytes)
+    for _ in range(3):
+        assert torch.equal(_run_ffn(plan, x, w1, w2, hidden, pool.data_ptr()), expected)
+        assert bool((pool[words:] == GUARD).all()) and counters_are_zero(plan, pool)
+
+
+@pytest.mark.parametrize("m, k, h, n", [
+    (8, 6784, 11648, 320),
+    (1, 512, 6161, 512),        # uneven pieces, two slots a workgroup
+    (128, 4096, 16384, 4096),
+    (3, 7552, 3328, 3712),      # both GEMMs split
+])
+def test_split_basic_down_from_dirty_counters(m, k, h, n):
+    """A split Basic down through ffn_mi355x_run starts right from whatever its counters held (the up
+    launch clears them), stays inside plan.workspace_bytes and leaves the counters zero."""
+    plan = _lib.make_plan(_align(m, 64), _align(k, 16), _align(h, 64), _align(n, 64), _lib.BF16, "basic", "erf", 256,
+                          m=m)
+    assert plan.down_sk_tiles > 0
+    x, w1, w2, hidden = _ffn_operands(m, k, h, n, plan)
+    clean = poisoned_workspace(plan)
+    expected = _run_ffn(plan, x, w1, w2, hidden, clean.data_ptr())
+    assert not bool(expected[:m, :n].isnan().any())
+    pool = torch.full((32 << 20,), GUARD, dtype=torch.int32, device="cuda")
+    words = plan.workspace_bytes // 4
+    pool[:words] = poisoned_workspace(plan).view(torch.int32)
+    stride = 32 if (plan.up_sk_tiles + plan.down_sk_tiles) * 32 * 4 <= 64 << 10 else 1
+    down_words = plan.down_sk_tiles * stride
+    say("dirty", m, k, h, n, plan.up_sk_tiles, plan.down_sk_tiles)
+    for garbage in (1, 0x7FFFFFFF, -1):
+        pool[:down_words] = garbage
+        assert torch.equal(_run_ffn(plan, x, w1, w2, hidden, pool.data_ptr()), expected)
+        assert bool((pool[words:] == GUARD).all()) and counters_are_zero(plan, pool)
+    # and without a workspace: whole tiles of the same size.  Both round an FP32 sum to bf16 (half an ulp,
+    # 2^-9 of the value, each), and the sums' own difference is far below that: 2^-7 of the largest value
+    if plan.up_sk_tiles == 0:
+        whole = _run_ffn(plan, x, w1, w2, hidden, None)
+        scale = expected[:m, :n].float().abs().max()
+        assert float((whole[:m, :n].float() - expected[:m, :n].float()).abs().max()) <= float(scale) * 2 ** -7

@@ -798,6 +798,76 @@ def test_large_block_num_never_refuses_a_basic_plan(block_num):
             assert p.workspace_bytes < 1 << 31
 
 
+def _c_plan(m, k, h, n, down="basic", block_num=256, down_variant=-1):
+    """A plan as a C caller gets it from ffn_mi355x_make_plan alone."""
+    plan = _lib.PlanStruct()
+    a64 = lambda v: -(-v // 64) * 64
+    _lib.check(_lib.load().ffn_mi355x_make_plan(m, a64(m), -(-k // 16) * 16, a64(h), a64(n), _lib.BF16,
+                                                _lib.DOWN_CODES[down], 0, block_num, -1, down_variant,
+                                                ctypes.byref(plan)))
+    return plan
+
+
+@pytest.mark.parametrize("m, k, h, n, up_split", [
+    (8, 6784, 11648, 320, False),      # whose split down would write 393216 bytes of workspace
+    (3, 4832, 7232, 640, False),
+    (128, 4096, 16384, 4096, False),
+    (3, 7552, 3328, 3712, True),       # the split up's workspace alone
+    (16, 5120, 13824, 5120, False),
+    (512, 1024, 4096, 1024, False),
+])
+def test_basic_down_is_split_only_when_asked(m, k, h, n, up_split):
+    """ffn_mi355x_make_plan plans whole down tiles: a caller's `ws` is not written by them, whatever it
+    points to, and workspace_bytes covers no split nobody asked for.  ffn_mi355x_set_split_down turns the
+    split on, with the bytes it needs, and off again."""
+    lib = _lib.load()
+    plan = _c_plan(m, k, h, n)
+    assert (plan.up_sk_tiles > 0) == up_split
+    assert plan.down_sk_tiles == plan.down_slots_per_wg == 0 and plan.down_dp_tiles == plan.down_tiles
+    assert plan.down_grid == min(plan.down_tiles, 256)
+    up_bytes = plan.up_grid * plan.up_slots_per_wg * plan.up_bm * plan.up_bn * 4 if up_split else 0
+    counters = _lib.workspace_counter_bytes(plan)
+    assert plan.workspace_bytes == up_bytes + counters and (counters > 0) == up_split
+    whole = bytes(plan)
+    _lib.set_operands(plan, k, h, n, k, k, h)
+    _lib.check(lib.ffn_mi355x_set_split_down(ctypes.byref(plan), 1, -1))
+    assert plan.down_sk_tiles == plan.down_tiles > 0 and plan.down_dp_tiles == 0
+    need = plan.down_grid * plan.down_slots_per_wg * plan.down_bm * plan.down_bn * 4
+    assert plan.workspace_bytes >= need + _lib.workspace_counter_bytes(plan) > need
+    assert (plan.k, plan.h, plan.n, plan.ldx, plan.ldw1, plan.ldw2) == (k, h, n, k, k, h)
+    host = _lib.make_plan(plan.mp, plan.kp, plan.hp, plan.np, _lib.BF16, "basic", "erf", 256, m=m)
+    _lib.set_operands(host, k, h, n, k, k, h)
+    assert bytes(host) == bytes(plan)      # the Python host, which owns its workspace, asks for the split
+    _lib.check(lib.ffn_mi355x_set_split_down(ctypes.byref(plan), 0, -1))
+    _lib.set_operands(plan, plan.kp, plan.hp, plan.np, plan.kp, plan.kp, plan.hp)
+    assert bytes(plan) == whole
+    assert bytes(_lib.make_plan(plan.mp, plan.kp, plan.hp, plan.np, _lib.BF16, "basic", "erf", 256, m=m,
+                                split_down=False)) == whole
+
+
+def test_set_split_down_refusals_leave_the_plan():
+    lib = _lib.load()
+    streamk = _c_plan(16, 5120, 13824, 5120, "streamk")
+    single = _c_plan(4096, 1024, 4096, 1024, down_variant=21)
+    pair = _lib.make_plan(4096, 1024, 4096, 1024, _lib.BF16, "basic", "erf", 256, 12, 21)
+    _lib.set_single_launch(pair, True)
+    for plan, variant, code in ((streamk, -1, _lib.ENOT_APPLICABLE), (pair, -1, _lib.ENOT_APPLICABLE),
+                                (single, lib.ffn_mi355x_num_variants(), _lib.EINVAL)):
+        before = bytes(plan)
+        assert lib.ffn_mi355x_set_split_down(ctypes.byref(plan), 1, variant) == code and _lib.last_error()
+        assert bytes(plan) == before
+    single.down_tiles += 1
+    assert lib.ffn_mi355x_set_split_down(ctypes.byref(single), 1, -1) == _lib.EINVAL
+    assert lib.ffn_mi355x_set_split_down(None, 1, -1) == _lib.EINVAL
+
+
+def test_set_split_down_keeps_whole_tiles_where_they_fill_the_grid():
+    plan = _c_plan(4096, 1024, 4096, 1024)
+    whole = bytes(plan)
+    _lib.check(_lib.load().ffn_mi355x_set_split_down(ctypes.byref(plan), 1, -1))
+    assert bytes(plan) == whole and plan.down_sk_tiles == 0
+
+
 def test_swiglu_up_takes_narrow_tiles_at_small_m():
     """SwiGLU up tiles at few rows: 64x64 where 128 columns leave CUs idle (12.9 -> 10.4 us), and
     64 rows rather than 128 of which half hold no data (44.6 -> 37.7 us)."""
