@@ -115,8 +115,9 @@ def prepare_ffn(x, weight1, weight2, *, up_impl="basic", down_impl="basic", bloc
     cu_count, _arch = _lib.query(device)
     if block_num is None:
         block_num = cu_count
+    # the single launch runs whole down tiles: its plan picks the down's tile among those
     plan = make_plan(p, selection, block_num, gelu=gelu, up_variant=up_variant,
-                     down_variant=down_variant)
+                     down_variant=down_variant, split_down=not single_launch)
     if block_num > cu_count:
         raise ValueError(f"block_num must not exceed the device CU count ({cu_count})")
     if single_launch is not None:

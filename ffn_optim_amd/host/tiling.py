@@ -112,14 +112,15 @@ def _tile(bm, bn, bk, variant):
 
 
 def make_plan(problem, selection=Selection(), block_num=DEFAULT_BLOCK_NUM, *, gelu="erf",
-              up_variant=None, down_variant=None, tuned=True):
+              up_variant=None, down_variant=None, tuned=True, split_down=True):
     """Plan one FFN (ops/host/tiling.py:58-74).
 
     Raises DependencyUnavailable for full_load_*, ValueError for a block_num outside
     [1, 65535], NotApplicable when Stream-K has no remainder tiles for this
     block_num or H spans fewer than two K iterations.  With neither variant forced
     and tuned=True, a measured choice from the tuning table (ffn_optim_amd.tuning)
-    replaces the library planner's for the shapes it covers.
+    replaces the library planner's for the shapes it covers.  split_down=False keeps a Basic
+    down on whole tiles (what the single launch runs).
     """
     selection.require_available()
     if type(block_num) is not int or not 1 <= block_num <= 65535:
@@ -140,7 +141,7 @@ def make_plan(problem, selection=Selection(), block_num=DEFAULT_BLOCK_NUM, *, ge
     native = _lib.make_plan(mp, kp, hp, np_, dtype, selection.down_impl, gelu, block_num,
                             -1 if up_variant is None else up_variant,
                             -1 if down_variant is None else down_variant, m=problem.m,
-                            activation=activation)
+                            activation=activation, split_down=split_down)
     up = _tile(native.up_bm, native.up_bn, native.up_bk, native.up_variant)
     down = _tile(native.down_bm, native.down_bn, native.down_bk, native.down_variant)
     if native.workspace_bytes:   # split down and/or split up GEMM

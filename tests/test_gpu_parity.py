@@ -700,3 +700,20 @@ def test_single_launch_matches_two_launches(case_id, upv, downv):
         assert not bool(words.any()), words.nonzero()[:8]   # error word included
     if case_id == "c2_aligned_bf16":
         assert_parity(got, x, w1, w2, tag="single launch c2")
+
+
+def test_single_launch_with_an_automatic_down_tile():
+    """prepare_ffn(single_launch=True) picks the down's tile among those the single launch runs, also
+    for an FFN whose two launches would split another tile."""
+    gen = torch.Generator(device="cuda").manual_seed(29)
+    x = torch.randn((1469, 2688), generator=gen, device="cuda").bfloat16()
+    w1 = (torch.randn((4864, 2688), generator=gen, device="cuda") * 2688 ** -0.5).bfloat16()
+    w2 = (torch.randn((512, 4864), generator=gen, device="cuda") * 4864 ** -0.5).bfloat16()
+    say("single launch, automatic down")
+    one = prepare_ffn(x, w1, w2, up_variant=13, single_launch=True)
+    two = prepare_ffn(x, w1, w2, up_variant=13, down_variant=one.plan.down.variant, single_launch=True)
+    assert one.plan.native.single_launch == two.plan.native.single_launch == 1
+    got, want = one.run().clone(), two.run()
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    assert_parity(got, x, w1, w2, tag="single launch, automatic down")

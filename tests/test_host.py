@@ -868,6 +868,17 @@ def test_set_split_down_keeps_whole_tiles_where_they_fill_the_grid():
     assert bytes(plan) == whole and plan.down_sk_tiles == 0
 
 
+@pytest.mark.parametrize("m, k, h, n", [(1469, 2688, 4864, 512), (923, 1440, 22528, 448), (4197, 208, 6400, 128)])
+def test_single_launch_plans_keep_the_whole_tile_down(m, k, h, n):
+    """A plan for the single launch picks its down tile among whole tiles: one priced split (another
+    tile, without a single-launch kernel) would make it inapplicable."""
+    p = problem_from_shapes((m, k), (h, k), (n, h), "bfloat16")
+    plan = make_plan(p, Selection("basic", "basic"), 256, up_variant=13, split_down=False).native
+    assert plan.down_variant == 19 and plan.down_sk_tiles == 0
+    _lib.set_single_launch(plan, True)
+    assert make_plan(p, Selection("basic", "basic"), 256, up_variant=13).native.down_variant != 19
+
+
 def test_swiglu_up_takes_narrow_tiles_at_small_m():
     """SwiGLU up tiles at few rows: 64x64 where 128 columns leave CUs idle (12.9 -> 10.4 us), and
     64 rows rather than 128 of which half hold no data (44.6 -> 37.7 us)."""
