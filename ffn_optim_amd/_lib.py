@@ -195,24 +195,27 @@ def make_plan(mp, kp, hp, np_, dtype, down_impl, gelu, block_num, up_variant=-1,
               down_variant=-1, m=None, activation="gelu", split_down=True) -> PlanStruct:
     """Native plan; `m` is the logical row count (default: all mp rows hold data); `gelu` is the
     GELU form when activation is 'gelu'; split_down lets a Basic down split its tiles
-    (ffn_mi355x_set_split_down), for callers that allocate the plan's workspace_bytes.  A key
-    planned before returns a copy of its plan (the plan is a function of the arguments alone); at
-    most MAX_PLANS are kept."""
+    (ffn_mi355x_set_split_down), for callers that allocate the plan's workspace_bytes.  A key of
+    ints planned before returns a copy of its plan (the plan is a function of the arguments alone);
+    at most MAX_PLANS are kept.  Other arguments go to the library each time: a float equal to
+    a known int must be refused as ever, and a ctypes object may change."""
     lib = load()
     args = (mp if m is None else m, mp, kp, hp, np_, dtype, DOWN_CODES[down_impl],
             activation_code(activation, gelu), block_num, up_variant, down_variant)
     split_down = bool(split_down) and DOWN_CODES[down_impl] == DOWN_CODES["basic"]
+    key = (args, split_down) if all(type(a) is int for a in args) else None
     plans = memo(lib).setdefault("plans", {})
-    known = plans.get((args, split_down))
+    known = plans.get(key) if key is not None else None
     if known is not None:
         return PlanStruct.from_buffer_copy(known)
     plan = PlanStruct()
     check(lib.ffn_mi355x_make_plan(*args, ctypes.byref(plan)))
     if split_down and "ffn_mi355x_set_split_down" not in lib._ffn_missing_launch:
         check(lib.ffn_mi355x_set_split_down(ctypes.byref(plan), 1, down_variant))
-    if len(plans) >= MAX_PLANS:
-        plans.clear()
-    plans[args, split_down] = bytes(plan)
+    if key is not None:
+        if len(plans) >= MAX_PLANS:
+            plans.clear()
+        plans[key] = bytes(plan)
     return plan
 
 

@@ -879,6 +879,24 @@ def test_single_launch_plans_keep_the_whole_tile_down(m, k, h, n):
     assert make_plan(p, Selection("basic", "basic"), 256, up_variant=13).native.down_variant != 19
 
 
+def test_known_plans_do_not_change_what_make_plan_accepts():
+    """A plan kept for a key of ints answers that key alone: a float is refused whether or not its int
+    was planned before, and a ctypes integer is read at every call."""
+    def plan(up, down=5):
+        return _lib.make_plan(1024, 1024, 1024, 1024, _lib.BF16, "basic", "erf", 256, up, down)
+    assert plan(5).up_variant == 5 and plan(5) is not plan(5)
+    for bad in (5.0, "5"):
+        with pytest.raises(ctypes.ArgumentError):
+            plan(bad)
+    value = ctypes.c_int(5)
+    assert plan(value).up_variant == 5
+    value.value = 9
+    assert plan(value).up_variant == 9
+    first = plan(5)
+    first.up_variant = 3           # a copy: the kept plan is not reached through it
+    assert plan(5).up_variant == 5
+
+
 def test_swiglu_up_takes_narrow_tiles_at_small_m():
     """SwiGLU up tiles at few rows: 64x64 where 128 columns leave CUs idle (12.9 -> 10.4 us), and
     64 rows rather than 128 of which half hold no data (44.6 -> 37.7 us)."""
