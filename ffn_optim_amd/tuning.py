@@ -41,12 +41,15 @@ def _key_tuple(key: dict) -> tuple:
 
 
 def load(path: Path | str | None = None) -> dict:
-    """{key tuple: entry} of a table file; an absent file is an empty table."""
-    path = TABLE_PATH if path is None else Path(path)
+    """{key tuple: entry} of a table file (default: the package's); an absent file is an empty table,
+    one that cannot be looked at is an error."""
+    path = Path(path) if path else TABLE_PATH
     with _lock:
         try:
             mtime = os.stat(path).st_mtime
-        except OSError:
+        except (OSError, ValueError):
+            if path.exists():  # (raises where the directory may not be read)
+                raise
             mtime = None
         cached = _cache.get(path)
         if cached is not None and cached["mtime"] == mtime:

@@ -323,6 +323,23 @@ def test_committed_tuning_table_plans_every_entry():
                 assert tuning.lookup(key) == (plan.up.variant, plan.down.variant), (case["case_id"], down)
 
 
+def test_tuning_table_path_forms(tmp_path, monkeypatch):
+    """An empty path is the package's table; a path that cannot name a file is an empty table, and a
+    file that cannot be looked at an error rather than an empty table."""
+    import os
+    from ffn_optim_amd import tuning
+    assert tuning.load("") == tuning.load(None) == tuning.load(str(tuning.TABLE_PATH)) != {}
+    assert tuning.load(tmp_path / "absent.json") == tuning.load("a\0b") == {}
+    assert tuning.load(str(tuning.TABLE_PATH) + "/below") == {}
+
+    def refused(path, *args, **kwargs):
+        raise PermissionError(13, "Permission denied", str(path))
+    monkeypatch.setattr(os, "stat", refused)
+    monkeypatch.setattr(type(tmp_path), "stat", refused)
+    with pytest.raises(PermissionError):
+        tuning.load(tmp_path / "table.json")
+
+
 def test_tuning_table_rejects_bad_entries(tmp_path):
     from ffn_optim_amd import tuning
     bad = tmp_path / "bad.json"
