@@ -203,7 +203,7 @@ def make_plan(mp, kp, hp, np_, dtype, down_impl, gelu, block_num, up_variant=-1,
     args = (mp if m is None else m, mp, kp, hp, np_, dtype, DOWN_CODES[down_impl],
             activation_code(activation, gelu), block_num, up_variant, down_variant)
     split_down = bool(split_down) and DOWN_CODES[down_impl] == DOWN_CODES["basic"]
-    key = (args, split_down) if all(type(a) is int for a in args) else None
+    key = (args, split_down) if {*map(type, args)} == {int} else None
     plans = memo(lib).setdefault("plans", {})
     known = plans.get(key) if key is not None else None
     if known is not None:

@@ -139,7 +139,8 @@ def prepare_ffn(x, weight1, weight2, *, up_impl="basic", down_impl="basic", bloc
             start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             start.record()
         storage, layout, x_rows = prepare_storage(x, weight1, weight2, plan, alias_aligned=_alias,
-                                                  bias1=bias1, bias2=bias2)
+                                                  bias1=bias1, bias2=bias2,
+                                                  stream=None if timed else stream)
         if timed:
             end.record()
         _lib.set_operands(plan.native, *layout)
@@ -159,6 +160,8 @@ def ffn(x, weight1, weight2, **configuration):
     Operands the kernels can read where they lie (contiguous, rows a multiple of 8
     elements: K for X and weight1, H for weight2) are used in place for this single
     launch instead of being copied into padded buffers; the result is identical (the
-    kernels zero-fill past the logical widths and mask ragged tiles).
+    kernels zero-fill past the logical widths and mask ragged tiles).  The call does not wait:
+    copies and launches read the operands in the order of the current stream, like any
+    asynchronous torch operator.
     """
     return prepare_ffn(x, weight1, weight2, **configuration, _alias=True).run()

@@ -208,7 +208,7 @@ def _padded(src, rows, cols, clean_rows):
     return out
 
 
-def prepare_storage(x, weight1, weight2, plan, alias_aligned=False, bias1=None, bias2=None):
+def prepare_storage(x, weight1, weight2, plan, alias_aligned=False, bias1=None, bias2=None, stream=None):
     """Contiguise and zero-pad into [mp,kp], [hp,kp], [np,hp]; allocate hidden, out, workspace.
 
     Same buffers as ops/host/inputs.py:74-90; the FP32 workspace holds the arrival counters and
@@ -223,6 +223,10 @@ def prepare_storage(x, weight1, weight2, plan, alias_aligned=False, bias1=None, 
     in place even as a permuted or sliced view (row_grid); W1 needs K % 8 == 0 and W2
     H % 8 == 0, both contiguous (a transposed weight is copied).  X read in place is kept as
     an [m, k] view at pitch ldx, or as the caller's tensor itself when its rows form a grid.
+
+    stream: the current stream, where the call returns before the copies on it have run.  The
+    caller may drop a copied operand then, and its memory stays until they have, also where it
+    was allocated on another stream.
     """
     import torch
 
@@ -239,6 +243,7 @@ def prepare_storage(x, weight1, weight2, plan, alias_aligned=False, bias1=None, 
         ws.view(-1)[:_lib.workspace_counter_bytes(native) // 4].zero_()
     grid = row_grid(x, p.k) if alias_aligned else None
     x_rows = None
+    copied = []
     if grid is not None and grid[0] == "pitch":
         ldx = grid[1]
         xs = x.as_strided((p.m, p.k), (ldx, 1))
@@ -247,19 +252,23 @@ def prepare_storage(x, weight1, weight2, plan, alias_aligned=False, bias1=None, 
     else:
         xs = _padded(x.reshape(p.m, p.k), plan.mp, plan.kp, not alias_aligned)
         ldx = plan.kp
+        copied.append(x)
     if p.activation == "swiglu":
         # always a copy: the gate and up rows are interleaved for the up GEMM
         w1s, ldw1 = interleave_gate_up(weight1, p.h, plan.hp, plan.kp), plan.kp
+        copied.append(weight1)
     elif alias_aligned and _in_place(weight1, p.k):
         w1s, ldw1 = weight1, p.k
     else:
         w1s = _padded(weight1, plan.hp, plan.kp, not alias_aligned)
         ldw1 = plan.kp
+        copied.append(weight1)
     if alias_aligned and _in_place(weight2, p.h):
         w2s, ldw2 = weight2, p.h
     else:
         w2s = _padded(weight2, plan.np, plan.hp, not alias_aligned)
         ldw2 = plan.hp
+        copied.append(weight2)
     # the reduction runs to the logical K when both up operands hold whole chunks up to it
     k = p.k if p.k % 8 == 0 else plan.kp
     layout = (k, p.h, p.n, ldx, ldw1, ldw2)
@@ -269,6 +278,10 @@ def prepare_storage(x, weight1, weight2, plan, alias_aligned=False, bias1=None, 
         b1s = (interleave_gate_up(bias1, p.h, plan.hp) if p.activation == "swiglu"
                else bias1.detach().clone().contiguous())
         storage += (b1s, bias2.detach().clone().contiguous())
+        copied += [bias1, bias2]
+    if stream is not None:
+        for t in copied:
+            t.record_stream(stream)
     return storage, layout, x_rows
 
 

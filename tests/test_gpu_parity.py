@@ -594,6 +594,32 @@ def test_streamk_finish_reproducible_and_resets(dtype):
     assert 2 in pieces_seen and max(pieces_seen) >= 3   # tiles of two pieces and of three or more
 
 
+@pytest.mark.parametrize("activation", ["gelu", "swiglu"])
+def test_one_shot_operands_of_another_stream_may_be_dropped(activation):
+    """A one-shot call on a busy side stream returns before its operands are copied.  Operands allocated
+    on the default stream and dropped right after the call keep their memory until then: new tensors
+    of the default stream do not overwrite them."""
+    from ffn_optim_amd import eagle_ffn_linear
+    m, k, h, n = 37, 1001, 771, 333     # odd widths: every operand is copied
+    u = 2 * h if activation == "swiglu" else h
+    gen = torch.Generator(device="cuda").manual_seed(31)
+    shapes = ((m, k), (u, k), (n, h), (u,), (n,))
+    kept = [(torch.randn(s, generator=gen, device="cuda") * 0.05).bfloat16() for s in shapes]
+    want = eagle_ffn_linear(*kept, activation).clone()
+    operands = [t.clone() for t in kept]
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    say("dropped operands", activation)
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(200_000_000)     # about 0.1 s
+        got = eagle_ffn_linear(*operands, activation)
+    del operands
+    over = [torch.full(s, 7.0, dtype=torch.bfloat16, device="cuda") for s in shapes]
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    del over
+
+
 @pytest.mark.parametrize("fill", [0xFFFFFFFF, 7, "random"])
 def test_dirty_counter_region_is_repaired(fill):
     """The workspace's arrival counters need not start at zero for a Stream-K down after its up
