@@ -234,6 +234,14 @@ bool sk_shape(const Variant& v, long long m_valid, long long N, long long K, int
     return s.sk > 0 && s.k_iters >= 2 && counters_fit(s.sk, v);
 }
 
+// Latency of a shared tile's finish (seconds) at p pieces: write-through, arrival count, reads, store.
+double finish_latency(const Variant& v, double p) {
+    return 1.0e-6 + 0.4e-6 * p + (double)v.bm * v.bn * 4.0 * (24e-12 + 5e-12 * p);
+}
+
+// Pieces that do not cut a tile's iterations evenly run on from one tile into the next.
+bool uneven(const SkShape& s) { return s.pieces > 0 && s.k_iters % s.pieces != 0; }
+
 double cost_streamk(const Variant& v, const SkShape& s, long long m_valid, long long N, long long K,
                     bool up = false) {
     const long long G = s.grid;
@@ -261,10 +269,9 @@ double cost_streamk(const Variant& v, const SkShape& s, long long m_valid, long 
     const long long pieces_per_tile =
         s.pieces ? s.pieces : std::min<long long>(G, cdiv(s.k_iters, std::max<long long>(1, s.q)) + 1);
     if (s.k_iters > sk_iters) {
-        const double tile_bytes = (double)v.bm * v.bn * 4.0, p = (double)pieces_per_tile;
-        const double latency = 1.0e-6 + 0.4e-6 * p + tile_bytes * (24e-12 + 5e-12 * p);
-        const double traffic = (double)s.sk * (2.0 * p - 1.0) * tile_bytes / kPartialRate;
-        t += std::max(latency * (scattered ? 2.0 : 1.0), traffic);
+        const double p = (double)pieces_per_tile;
+        const double traffic = (double)s.sk * (2.0 * p - 1.0) * (double)v.bm * v.bn * 4.0 / kPartialRate;
+        t += std::max(finish_latency(v, p) * (scattered ? 2.0 : 1.0), traffic);
     }
     const double hbm = (double)(N * K + m_valid * K) * 2.0 / kHbmRate;
     return std::max(t, hbm);
@@ -285,8 +292,8 @@ bool better(double c, const Variant& v, double best_cost, const Variant& best, l
 // A GEMM with every tile split along K: open to tiles that would leave at least half of the
 // workgroups idle and a reduction deep enough to split (a decode-size FFN with a narrow H, e.g. one
 // GPU's H/8 share of a 16x5120 -> 13824 FFN, whose few up tiles would stream W1 on a few CUs).
-// Every tile is then cut into p equal pieces (sk_grid); the last piece of a tile to finish sums the
-// partials and stores the tile (the up GEMM's applies the activation).  On that decode shard (54
+// Every tile is then cut into p pieces (sk_grid; equal where p divides its iterations); the last piece
+// of a tile to finish sums the partials and stores the tile (the up GEMM's applies the activation).  On that decode shard (54
 // up tiles of 32x32, 4 pieces of 10 iterations on 216 workgroups) the split up takes 8.9 us.
 constexpr int kSplitMinIters = 16;
 bool split_whole(const Variant& v, long long m_valid, long long N, long long K, int G, SkShape& s) {
@@ -322,13 +329,13 @@ constexpr long long kUnevenMinIters = 48;
 // split; 368 rows, 512 -> 3584 down: 17.0 and 17.3).
 constexpr double kSplitMargin = 1.1;
 double split_price(const Variant& v, const SkShape& s, long long m_valid, long long N, long long K, bool up = false) {
-    return cost_streamk(v, s, m_valid, N, K, up) * (s.k_iters % s.pieces == 0 ? kSplitMargin : kUnevenPieces);
+    return cost_streamk(v, s, m_valid, N, K, up) * (uneven(s) ? kUnevenPieces : kSplitMargin);
 }
 bool split_down(const Variant& v, long long M, long long m_valid, long long N, long long K, int G, SkShape& s,
                 double& cost) {
     cost = cost_basic(v, M, m_valid, N, K, G);
     if (K < kSplitDownMinK || !split_whole(v, m_valid, N, K, G, s)) return false;
-    if (s.k_iters % s.pieces != 0 && (s.k_iters < kUnevenMinIters || (s.pieces > 2 && 2 * s.grid > G))) return false;
+    if (uneven(s) && (s.k_iters < kUnevenMinIters || (s.pieces > 2 && 2 * s.grid > G))) return false;
     const double c = split_price(v, s, m_valid, N, K);
     if (c >= cost) return false;
     cost = c;
@@ -355,6 +362,15 @@ int pick_basic(long long M, long long m_valid, long long N, long long K, int G, 
 // than the whole tiles it replaces.  A forced down_variant still takes it.
 bool sk_candidate(const Variant& v) { return !(v.mf == 16 && v.bn == 192); }
 
+// A Stream-K tile in uneven pieces pays for a second unit and a second finish in most workgroups
+// (over 121 of them timed, 3-7 us more than even pieces of the same price): 128 rows, 1359 -> 1762,
+// 112 pieces of K-sliced 64x64 tiles 64 deep, 11 iterations each: FFN 15.5 us, uneven 128-deep ones
+// 21.0; 176 rows, 3657 -> 2560: 23.7 and 27.4; 1600 rows, 7348 -> 3328, 256x256: 196.5 and 200.4.
+// Over 70 FFNs whose pick this moves: 1.13 times faster on average, 0.94 at worst.
+double price_streamk(const Variant& v, const SkShape& s, long long m_valid, long long N, long long K) {
+    return cost_streamk(v, s, m_valid, N, K) + (uneven(s) ? kUnitOverhead + finish_latency(v, (double)s.pieces) : 0.0);
+}
+
 int pick_streamk(long long M, long long m_valid, long long N, long long K, int G) {
     int best = -1;
     double best_cost = 1e300;
@@ -362,7 +378,7 @@ int pick_streamk(long long M, long long m_valid, long long N, long long K, int G
         if (!sk_candidate(kVariants[i])) continue;
         SkShape s;
         if (!sk_shape(kVariants[i], m_valid, N, K, G, s)) continue;
-        const double c = cost_streamk(kVariants[i], s, m_valid, N, K);
+        const double c = price_streamk(kVariants[i], s, m_valid, N, K);
         if (best < 0 || better(c, kVariants[i], best_cost, kVariants[best], m_valid)) best_cost = c, best = i;
     }
     return best;

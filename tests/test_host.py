@@ -897,6 +897,19 @@ def test_known_plans_do_not_change_what_make_plan_accepts():
     assert plan(5).up_variant == 5
 
 
+@pytest.mark.parametrize("m, k, h, n, even", [
+    (176, 2560, 3657, 2560, 14),     # 58 iterations of 64 in two; 29 of 128 do not halve
+    (496, 4992, 863, 512, 14),
+    (1699, 1984, 1800, 4167, 6),     # 58 of 32 against 29 of 64
+])
+def test_streamk_pick_prefers_even_pieces(m, k, h, n, even):
+    """Among near ties the automatic Stream-K down takes the tile whose pieces cut its iterations evenly."""
+    p = problem_from_shapes((m, k), (h, k), (n, h), "bfloat16")
+    native = make_plan(p, Selection("basic", "streamk"), 256, tuned=False).native
+    assert native.down_variant == even
+    assert native.down_k_iters % (native.down_grid // native.down_sk_tiles) == 0
+
+
 def test_swiglu_up_takes_narrow_tiles_at_small_m():
     """SwiGLU up tiles at few rows: 64x64 where 128 columns leave CUs idle (12.9 -> 10.4 us), and
     64 rows rather than 128 of which half hold no data (44.6 -> 37.7 us)."""
