@@ -283,10 +283,14 @@ double cost_streamk(const Variant& v, const SkShape& s, long long m_valid, long 
 // instead of the lower variant number (aligned mid-size down at 2048 rows: v24 133.3 us, v18
 // 147.7, v10 155.0, one tuning run).  Not where the tiles are taller than the rows holding data:
 // a decode-size GEMM at the HBM bound gains nothing from a tall tile's efficiency (16 x 8192 ->
-// 21824: the 128x128 tile 4% behind the 32x32 one).
-bool better(double c, const Variant& v, double best_cost, const Variant& best, long long m_valid) {
-    return c < best_cost * 0.999 || (c <= best_cost * 1.001 && v.bm <= m_valid && best.bm <= m_valid &&
-                                     tile_eff(v) > tile_eff(best));
+// 21824: the 128x128 tile 4% behind the 32x32 one).  Two forms of one tile shape tie there too: as the
+// down, the one with refill waves is ahead (K-sliced 32x32, 3 rows, 5120 -> 4864: FFN 18.9 us with
+// them, 20.6 without; 16 rows, 1800 -> 7186: 15.6 and 17.2; 102 rows, 128x128: 23.8 and 26.5); as the
+// up, 15 FFNs of 105 to 122 rows measured between 12% behind and 12% ahead.
+bool better(double c, const Variant& v, double best_cost, const Variant& best, long long m_valid, bool up = false) {
+    const bool same = !up && v.bm == best.bm && v.bn == best.bn && v.bk == best.bk && v.wgk == best.wgk;
+    return c < best_cost * 0.999 || (c <= best_cost * 1.001 && tile_eff(v) > tile_eff(best) &&
+                                     (same || (v.bm <= m_valid && best.bm <= m_valid)));
 }
 
 // A GEMM with every tile split along K: open to tiles that would leave at least half of the
@@ -416,7 +420,7 @@ int pick_up(long long M, long long m_valid, long long N, long long K, int G, boo
         if (split && fills) continue;
         const double c = split ? split_price(kVariants[i], s, m_valid, N, K, true)
                                : cost_basic(kVariants[i], M, m_valid, N, K, G, true);
-        if (best < 0 || better(c, kVariants[i], best_cost, kVariants[best], m_valid)) best_cost = c, best = i;
+        if (best < 0 || better(c, kVariants[i], best_cost, kVariants[best], m_valid, true)) best_cost = c, best = i;
     }
     return best;
 }

@@ -910,6 +910,14 @@ def test_streamk_pick_prefers_even_pieces(m, k, h, n, even):
     assert native.down_k_iters % (native.down_grid // native.down_sk_tiles) == 0
 
 
+@pytest.mark.parametrize("m, k, h, n", [(3, 424, 5120, 4864), (1, 768, 2328, 5120), (2, 4352, 4056, 4352)])
+def test_streamk_decode_tie_takes_the_refill_waves(m, k, h, n):
+    """Where the HBM term ties the two forms of the 32x32 tile, the one with refill waves is taken."""
+    p = problem_from_shapes((m, k), (h, k), (n, h), "bfloat16")
+    native = make_plan(p, Selection("basic", "streamk"), 256, tuned=False).native
+    assert native.down_variant == 20
+
+
 def test_swiglu_up_takes_narrow_tiles_at_small_m():
     """SwiGLU up tiles at few rows: 64x64 where 128 columns leave CUs idle (12.9 -> 10.4 us), and
     64 rows rather than 128 of which half hold no data (44.6 -> 37.7 us)."""
