@@ -127,7 +127,8 @@ constexpr double kUnitOverhead = 2.5e-6;   // s per unit: DMA prologue latency +
 // and unaligned up it serves.  A tile of 16x16x32 blocks runs at a higher clock for the same
 // power: the DiT-size up GEMM 7% and its Stream-K down 4% faster than on the same tile of
 // 32x32x16 blocks.
-double tile_eff(const Variant& v, bool up = false) {
+// former: as rated for the former Stream-K prices (plan_streamk).
+double tile_eff(const Variant& v, bool up = false, bool former = false) {
     const int a = v.bm < v.bn ? v.bm : v.bn, b = v.bm < v.bn ? v.bn : v.bm;
     const double refill = (v.prod > 0 ? 1.03 : 1.0) * (v.mf == 16 ? 1.05 : 1.0);
     // The K-sliced 32x32 decode tile (32x32 wave tiles, one MFMA per k-step and wave) reads the
@@ -135,7 +136,12 @@ double tile_eff(const Variant& v, bool up = false) {
     // FFN's Basic down: 512 tiles of it took 30.7 us against 27.0 us for 128 of 64x64, one tuning
     // run).  0.38 and 0.19 order the tiles of 32 FFN shapes timed in one run (16 to 4096 rows,
     // whole and split): the picks average 1% behind the fastest tile; at 0.3 and 0.15, 4%.
-    if (v.wgk > 1) return refill * (a >= 128 ? (v.nw + v.prod >= 8 ? 0.9 : 0.85) : a >= 64 ? (v.nw + v.prod >= 8 ? 0.38 : 0.34) : 0.19);
+    if (v.wgk > 1) {
+        const bool eight = v.nw + v.prod >= 8;
+        if (a >= 128) return refill * (eight ? 0.9 : 0.85);
+        if (former) return refill * (a >= 64 ? 0.3 : 0.15);
+        return refill * (a >= 64 ? (eight ? 0.38 : 0.34) : 0.19);
+    }
     if (a >= 256) return refill * 1.0;
     // 256x192 (16x16 blocks): 0.92 per FLOP of the 256x256 tile, from the DiT-size up at eight
     // tiles per CU (493.5 against 453.0 us at six of 256x256) and its H/8 shard at one wave of
@@ -153,9 +159,9 @@ double tile_eff(const Variant& v, bool up = false) {
 }
 
 // Seconds per BK-deep iteration of one workgroup on a tile with `rows` data-bearing rows.
-double iter_time(const Variant& v, long long rows, bool up = false) {
+double iter_time(const Variant& v, long long rows, bool up = false, bool former = false) {
     const double flops = 2.0 * v.bm * v.bn * v.bk;
-    const double t_mfma = flops / (kCuMfmaRate * tile_eff(v, up));
+    const double t_mfma = flops / (kCuMfmaRate * tile_eff(v, up, former));
     const double bytes = (double)(rows + v.bn) * v.bk * 2.0;
     const double inflight = (double)(v.stages - 1) * (double)(v.bm + v.bn) * v.bk * 2.0;
     // refill-only waves take the texture unit's stalls off the tile waves, where the refill
@@ -166,7 +172,7 @@ double iter_time(const Variant& v, long long rows, bool up = false) {
     // A tile of 128 rows or more with at most half of them holding data still reads its fragments and
     // issues its MFMAs for all of them (SwiGLU up, 16 rows, 4096 -> 11008, 172 tiles: 128x128 44.6 us,
     // 64x128 37.7).
-    const double idle_rows = v.bm >= 128 && 2 * rows <= v.bm ? 1.3 : 1.0;
+    const double idle_rows = !former && v.bm >= 128 && 2 * rows <= v.bm ? 1.3 : 1.0;
     return std::max(t_mfma, bytes / rate) * idle_rows;
 }
 
@@ -235,7 +241,12 @@ bool sk_shape(const Variant& v, long long m_valid, long long N, long long K, int
 }
 
 // Latency of a shared tile's finish (seconds) at p pieces: write-through, arrival count, reads, store.
-double finish_latency(const Variant& v, double p) {
+// former: with one partial load in flight per wave, or four for a wave of at most two 32x32 blocks.
+double finish_latency(const Variant& v, double p, bool former = false) {
+    if (former) {
+        const double per_read = (long long)v.bm * v.bn / v.nw <= 2048 ? 4.0 : 1.0;
+        return 1.2e-6 * (2.0 + std::ceil((p - 1.0) / per_read)) + p * (double)v.bm * v.bn * 4.0 / kCuLoadRate;
+    }
     return 1.0e-6 + 0.4e-6 * p + (double)v.bm * v.bn * 4.0 * (24e-12 + 5e-12 * p);
 }
 
@@ -243,9 +254,9 @@ double finish_latency(const Variant& v, double p) {
 bool uneven(const SkShape& s) { return s.pieces > 0 && s.k_iters % s.pieces != 0; }
 
 double cost_streamk(const Variant& v, const SkShape& s, long long m_valid, long long N, long long K,
-                    bool up = false) {
+                    bool up = false, bool former = false) {
     const long long G = s.grid;
-    const double it = iter_time(v, rows_in_tile(v, m_valid), up);
+    const double it = iter_time(v, rows_in_tile(v, m_valid), up, former);
     const long long dp_waves = cdiv(s.dp, G);
     const long long sk_iters = s.q + (s.r ? 1 : 0);
     // Pieces that start at scattered depths of their tiles (a grid of block_num workgroups over
@@ -266,12 +277,13 @@ double cost_streamk(const Variant& v, const SkShape& s, long long m_valid, long 
     // pieces: 2.9 us for 16 KiB tiles, 5.4 for 64, 13.5 for 256; two pieces: 2.0 and 4.2 us for 16
     // and 64), many the memory traffic of the partials (128 tiles of 256x192 in two pieces: 75 MB
     // in 31 us; 64 of 256x256 in four: 117 MB in 38-46); pieces that straddle tiles finish two.
-    const long long pieces_per_tile =
-        s.pieces ? s.pieces : std::min<long long>(G, cdiv(s.k_iters, std::max<long long>(1, s.q)) + 1);
+    // (the former prices count a piece more where the grid cuts every tile alike)
+    const long long pieces_per_tile = s.pieces && !former
+        ? s.pieces : std::min<long long>(G, cdiv(s.k_iters, std::max<long long>(1, s.q)) + 1);
     if (s.k_iters > sk_iters) {
         const double p = (double)pieces_per_tile;
         const double traffic = (double)s.sk * (2.0 * p - 1.0) * (double)v.bm * v.bn * 4.0 / kPartialRate;
-        t += std::max(finish_latency(v, p) * (scattered ? 2.0 : 1.0), traffic);
+        t += former ? finish_latency(v, p, true) : std::max(finish_latency(v, p) * (scattered ? 2.0 : 1.0), traffic);
     }
     const double hbm = (double)(N * K + m_valid * K) * 2.0 / kHbmRate;
     return std::max(t, hbm);
@@ -287,9 +299,11 @@ double cost_streamk(const Variant& v, const SkShape& s, long long m_valid, long 
 // down, the one with refill waves is ahead (K-sliced 32x32, 3 rows, 5120 -> 4864: FFN 18.9 us with
 // them, 20.6 without; 16 rows, 1800 -> 7186: 15.6 and 17.2; 102 rows, 128x128: 23.8 and 26.5); as the
 // up, 15 FFNs of 105 to 122 rows measured between 12% behind and 12% ahead.
-bool better(double c, const Variant& v, double best_cost, const Variant& best, long long m_valid, bool up = false) {
-    const bool same = !up && v.bm == best.bm && v.bn == best.bn && v.bk == best.bk && v.wgk == best.wgk;
-    return c < best_cost * 0.999 || (c <= best_cost * 1.001 && tile_eff(v) > tile_eff(best) &&
+bool better(double c, const Variant& v, double best_cost, const Variant& best, long long m_valid, bool up = false,
+            bool former = false) {
+    const bool same = !up && !former && v.bm == best.bm && v.bn == best.bn && v.bk == best.bk && v.wgk == best.wgk;
+    return c < best_cost * 0.999 || (c <= best_cost * 1.001 &&
+                                     tile_eff(v, false, former) > tile_eff(best, false, former) &&
                                      (same || (v.bm <= m_valid && best.bm <= m_valid)));
 }
 
@@ -375,15 +389,18 @@ double price_streamk(const Variant& v, const SkShape& s, long long m_valid, long
     return cost_streamk(v, s, m_valid, N, K) + (uneven(s) ? kUnitOverhead + finish_latency(v, (double)s.pieces) : 0.0);
 }
 
-int pick_streamk(long long M, long long m_valid, long long N, long long K, int G) {
+// The cheapest tile among those `ok` admits, -1 if none.  former: by the prices of the finish that kept
+// one partial load in flight a wave (plan_streamk).
+template <class Ok>
+int pick_streamk(long long m_valid, long long N, long long K, int G, bool former, const Ok& ok) {
     int best = -1;
     double best_cost = 1e300;
     for (int i = 0; i < kNumVariants; ++i) {
-        if (!sk_candidate(kVariants[i])) continue;
+        const Variant& v = kVariants[i];
         SkShape s;
-        if (!sk_shape(kVariants[i], m_valid, N, K, G, s)) continue;
-        const double c = price_streamk(kVariants[i], s, m_valid, N, K);
-        if (best < 0 || better(c, kVariants[i], best_cost, kVariants[best], m_valid)) best_cost = c, best = i;
+        if (!sk_candidate(v) || !sk_shape(v, m_valid, N, K, G, s) || !ok(v, s)) continue;
+        const double c = former ? cost_streamk(v, s, m_valid, N, K, false, true) : price_streamk(v, s, m_valid, N, K);
+        if (best < 0 || better(c, v, best_cost, kVariants[best], m_valid, false, former)) best_cost = c, best = i;
     }
     return best;
 }
@@ -614,6 +631,37 @@ bool fused_ok(const ffn_mi355x_plan* p) {
            ffn::kFusedReady + rbs * ffn::kFusedStride <= (long long)(kCounterBytes / 4) && fast_dma_for(p->kp);
 }
 
+// Whether a Stream-K down on tile v leaves a plan's workspace within `bytes` and its counters within
+// their region.
+bool streamk_fits(const ffn_mi355x_plan* p, const Variant& v, const SkShape& s, size_t bytes) {
+    const size_t words = (size_t)s.sk * v.nw + (size_t)p->up_sk_tiles * kVariants[p->up_variant].nw;
+    const size_t slots = (size_t)s.grid * s.slots * v.bm * v.bn * 4u;
+    return words <= kCounterBytes / 4 && std::max(slots, up_partial_bytes(p)) + kCounterBytes <= bytes;
+}
+
+// Automatic Stream-K tile: the cheapest, but no plan is refused, and none leaves the scratch of
+// ffn_mi355x_run_noalloc, on account of the prices having followed the faster finish.  They favour
+// larger tiles, whose partials outgrow that scratch or whose counters the region on about one FFN in
+// a thousand (132 rows, 15872 -> 4992: 15 MB on 64x128 tiles, 41 MB on 256x128, priced 2-6%
+// apart).  Where the former prices' tile fits a limit and the cheapest does not, the cheapest that fits
+// is taken.
+int plan_streamk(const ffn_mi355x_plan* p) {
+    const long long m = p->m, N = p->np, K = p->hp;
+    const int G = p->block_num;
+    int dv = pick_streamk(m, N, K, G, false, [](const Variant&, const SkShape&) { return true; });
+    if (dv < 0) return dv;
+    const int fv = pick_streamk(m, N, K, G, true, [](const Variant&, const SkShape&) { return true; });
+    for (const size_t limit : {((size_t)1 << 31) - 1, (size_t)FFN_MI355X_NOALLOC_SCRATCH_BYTES}) {
+        auto fits = [&](const Variant& v, const SkShape& s) { return streamk_fits(p, v, s, limit); };
+        auto tile_fits = [&](int i) {
+            SkShape s;
+            return sk_shape(kVariants[i], m, N, K, G, s) && fits(kVariants[i], s);
+        };
+        if (!tile_fits(dv) && tile_fits(fv)) dv = pick_streamk(m, N, K, G, false, fits);
+    }
+    return dv;
+}
+
 // Down GEMM of a plan whose up GEMM is planned, [mp x np], depth hp: its tile, its schedule and the
 // workspace of the two.  split: a Basic down may split its tiles (ffn_mi355x_set_split_down).
 int plan_down(ffn_mi355x_plan* plan, int down_variant, bool split) {
@@ -638,7 +686,7 @@ int plan_down(ffn_mi355x_plan* plan, int down_variant, bool split) {
             }
             dv = down_variant;
         } else {
-            dv = pick_streamk(mp, m, np, hp, G);
+            dv = plan_streamk(plan);
             if (dv < 0) {
                 bool any_two = false;
                 for (int i = 0; i < kNumVariants; ++i) any_two |= cdiv(hp, kVariants[i].bk) >= 2;

@@ -918,6 +918,23 @@ def test_streamk_decode_tie_takes_the_refill_waves(m, k, h, n):
     assert native.down_variant == 20
 
 
+@pytest.mark.parametrize("m, h, n, block_num", [
+    (132, 15872, 4992, 256),     # 15 MB of partials on 64x128 tiles, 41 MB on the 256x128 ones priced below
+    (187, 512, 8512, 256), (5083, 12032, 192, 256), (911, 6080, 13184, 64), (1166, 12800, 1088, 256),
+])
+def test_streamk_pick_keeps_the_noalloc_scratch(m, h, n, block_num):
+    """A faster finish moves automatic Stream-K downs to larger tiles, but not out of the scratch of
+    ffn_mi355x_run_noalloc, which held these plans' partials before."""
+    plan = _c_plan(m, 64, h, n, "streamk", block_num)
+    assert plan.down_sk_tiles > 0 and plan.workspace_bytes <= 32 << 20
+
+
+def test_streamk_pick_keeps_the_counter_region():
+    """Nor to a tile whose counters, beside those of a split up GEMM, outgrow their region."""
+    plan = _lib.make_plan(11840, 3696, 384, 6784, _lib.FP16, "streamk", "erf", 4096, 14, -1, m=11819)
+    assert plan.up_sk_tiles > 0 and plan.down_sk_tiles > 0
+
+
 def test_swiglu_up_takes_narrow_tiles_at_small_m():
     """SwiGLU up tiles at few rows: 64x64 where 128 columns leave CUs idle (12.9 -> 10.4 us), and
     64 rows rather than 128 of which half hold no data (44.6 -> 37.7 us)."""
