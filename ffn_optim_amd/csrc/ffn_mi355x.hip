@@ -385,8 +385,17 @@ bool sk_candidate(const Variant& v) { return !(v.mf == 16 && v.bn == 192); }
 // 112 pieces of K-sliced 64x64 tiles 64 deep, 11 iterations each: FFN 15.5 us, uneven 128-deep ones
 // 21.0; 176 rows, 3657 -> 2560: 23.7 and 27.4; 1600 rows, 7348 -> 3328, 256x256: 196.5 and 200.4.
 // Over 70 FFNs whose pick this moves: 1.13 times faster on average, 0.94 at worst.
+//
+// The large tiles of 32x32 blocks without refill waves are behind their price as Stream-K downs: over 37
+// FFNs the 128x256 one took 5% longer than the 256x128 one with refill waves where both were priced
+// alike, and near ties lost to it (5655 rows, 2560 -> 6144: FFN 310 us, on 128x256 328; 336 rows,
+// 2761 -> 5768: 65.2 and 68.7; 542 rows, 3755 -> 1072: on 64x64 36.2, on 45 tiles of 256x256 50.1).  Over
+// 60 FFNs whose pick this moves: 1.07 times faster on average, 0.94 at worst.
+constexpr double kPlainLargeTile = 1.06;
 double price_streamk(const Variant& v, const SkShape& s, long long m_valid, long long N, long long K) {
-    return cost_streamk(v, s, m_valid, N, K) + (uneven(s) ? kUnitOverhead + finish_latency(v, (double)s.pieces) : 0.0);
+    const bool plain = v.bm >= 128 && v.bn >= 128 && v.prod == 0 && v.mf == 32;
+    return cost_streamk(v, s, m_valid, N, K) * (plain ? kPlainLargeTile : 1.0) +
+           (uneven(s) ? kUnitOverhead + finish_latency(v, (double)s.pieces) : 0.0);
 }
 
 // The cheapest tile among those `ok` admits, -1 if none.  former: by the prices of the finish that kept

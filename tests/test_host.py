@@ -935,6 +935,13 @@ def test_streamk_pick_keeps_the_counter_region():
     assert plan.up_sk_tiles > 0 and plan.down_sk_tiles > 0
 
 
+@pytest.mark.parametrize("m, h, n", [(5655, 2560, 6144), (336, 2761, 5768), (1818, 768, 1464), (542, 3755, 1072)])
+def test_streamk_near_ties_do_not_take_large_tiles_without_refill_waves(m, h, n):
+    plan = _c_plan(m, 64, h, n, "streamk")
+    v = _lib.variants()[plan.down_variant]
+    assert v["refill_waves"] > 0 or v["mfma_edge"] == 16 or min(v["bm"], v["bn"]) < 128
+
+
 def test_swiglu_up_takes_narrow_tiles_at_small_m():
     """SwiGLU up tiles at few rows: 64x64 where 128 columns leave CUs idle (12.9 -> 10.4 us), and
     64 rows rather than 128 of which half hold no data (44.6 -> 37.7 us)."""
