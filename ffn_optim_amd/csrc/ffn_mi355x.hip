@@ -349,25 +349,45 @@ constexpr double kSplitMargin = 1.1;
 double split_price(const Variant& v, const SkShape& s, long long m_valid, long long N, long long K, bool up = false) {
     return cost_streamk(v, s, m_valid, N, K, up) * (uneven(s) ? kUnevenPieces : kSplitMargin);
 }
+// limit: what the split of a larger tile has to stay below (sliced_limit), for an automatic pick.
+constexpr double kNoLimit = 1e300;
 bool split_down(const Variant& v, long long M, long long m_valid, long long N, long long K, int G, SkShape& s,
-                double& cost) {
+                double& cost, double limit = kNoLimit) {
     cost = cost_basic(v, M, m_valid, N, K, G);
     if (K < kSplitDownMinK || !split_whole(v, m_valid, N, K, G, s)) return false;
     if (uneven(s) && (s.k_iters < kUnevenMinIters || (s.pieces > 2 && 2 * s.grid > G))) return false;
     const double c = split_price(v, s, m_valid, N, K);
-    if (c >= cost) return false;
+    if (c >= cost || (v.bm * v.bn > 64 * 64 && c >= limit)) return false;
     cost = c;
     return true;
 }
 
+// The K-sliced 64x64 tile is priced too high whole (512 rows, 4096 -> 1024: 13.4 us, priced 20.4; 256
+// rows, 8192 -> 2048: 22.6 and 38.2), as splits of larger tiles are not (15.8 and 16.6; 20.6 and 25.1).
+// Taken at those prices, 128x128 tiles in three or four pieces ahead of one wave of it were level over 64
+// FFNs, 0.82 to 1.20: below a depth of 9216 behind it more often than not (80 rows, 4608 -> 5376, 36.5 ->
+// 44.5 us; 2352 rows, 3840 -> 256, 30.5 -> 35.1), deeper mostly ahead (444 rows, 15360 -> 2304, 110 -> 85;
+// 684 rows, 9216 -> 1248, 53.9 -> 51.5).
+constexpr double kSlicedWhole = 0.8;
+constexpr long long kSlicedWholeMaxK = 9216;
+double sliced_limit(long long M, long long m_valid, long long N, long long K, int G) {
+    double limit = kNoLimit;
+    if (K >= kSlicedWholeMaxK) return limit;
+    for (const Variant& v : kVariants)
+        if (v.wgk > 1 && v.bm == 64 && v.bn == 64 && cdiv(m_valid, v.bm) * cdiv(N, v.bn) <= G)
+            limit = std::min(limit, kSlicedWhole * cost_basic(v, M, m_valid, N, K, G));
+    return limit;
+}
+
 // split: tiles are priced as split_down would run them, else whole.
 int pick_basic(long long M, long long m_valid, long long N, long long K, int G, bool split) {
+    const double limit = split ? sliced_limit(M, m_valid, N, K, G) : kNoLimit;
     int best = 0;
     double best_cost = 1e300;
     for (int i = 0; i < kNumVariants; ++i) {
         SkShape s;
         double c;
-        if (split) split_down(kVariants[i], M, m_valid, N, K, G, s, c);
+        if (split) split_down(kVariants[i], M, m_valid, N, K, G, s, c, limit);
         else c = cost_basic(kVariants[i], M, m_valid, N, K, G);
         if (better(c, kVariants[i], best_cost, kVariants[best], m_valid)) best_cost = c, best = i;
     }
@@ -709,7 +729,8 @@ int plan_down(ffn_mi355x_plan* plan, int down_variant, bool split) {
     } else {
         dv = down_variant >= 0 ? down_variant : pick_basic(mp, m, np, hp, G, split);
         double price;
-        split_basic = split && split_down(kVariants[dv], mp, m, np, hp, G, sb, price);
+        const double limit = down_variant >= 0 ? kNoLimit : sliced_limit(mp, m, np, hp, G);
+        split_basic = split && split_down(kVariants[dv], mp, m, np, hp, G, sb, price, limit);
         // whole tiles where a large block_num's pieces outgrow the counters or the 32-bit slot
         // offsets
         const size_t words = (size_t)sb.sk * kVariants[dv].nw +

@@ -732,9 +732,9 @@ def test_single_launch_with_an_automatic_down_tile():
     """prepare_ffn(single_launch=True) picks the down's tile among those the single launch runs, also
     for an FFN whose two launches would split another tile."""
     gen = torch.Generator(device="cuda").manual_seed(29)
-    x = torch.randn((1469, 2688), generator=gen, device="cuda").bfloat16()
-    w1 = (torch.randn((4864, 2688), generator=gen, device="cuda") * 2688 ** -0.5).bfloat16()
-    w2 = (torch.randn((512, 4864), generator=gen, device="cuda") * 4864 ** -0.5).bfloat16()
+    x = torch.randn((923, 1440), generator=gen, device="cuda").bfloat16()
+    w1 = (torch.randn((22528, 1440), generator=gen, device="cuda") * 1440 ** -0.5).bfloat16()
+    w2 = (torch.randn((448, 22528), generator=gen, device="cuda") * 22528 ** -0.5).bfloat16()
     say("single launch, automatic down")
     one = prepare_ffn(x, w1, w2, up_variant=13, single_launch=True)
     two = prepare_ffn(x, w1, w2, up_variant=13, down_variant=one.plan.down.variant, single_launch=True)

@@ -868,7 +868,7 @@ def test_set_split_down_keeps_whole_tiles_where_they_fill_the_grid():
     assert bytes(plan) == whole and plan.down_sk_tiles == 0
 
 
-@pytest.mark.parametrize("m, k, h, n", [(1469, 2688, 4864, 512), (923, 1440, 22528, 448), (4197, 208, 6400, 128)])
+@pytest.mark.parametrize("m, k, h, n", [(1343, 2496, 37632, 576), (923, 1440, 22528, 448), (4197, 208, 6400, 128)])
 def test_single_launch_plans_keep_the_whole_tile_down(m, k, h, n):
     """A plan for the single launch picks its down tile among whole tiles: one priced split (another
     tile, without a single-launch kernel) would make it inapplicable."""
@@ -940,6 +940,22 @@ def test_streamk_near_ties_do_not_take_large_tiles_without_refill_waves(m, h, n)
     plan = _c_plan(m, 64, h, n, "streamk")
     v = _lib.variants()[plan.down_variant]
     assert v["refill_waves"] > 0 or v["mfma_edge"] == 16 or min(v["bm"], v["bn"]) < 128
+
+
+@pytest.mark.parametrize("m, k, h, n, whole", [
+    (80, 5543, 4608, 5376, True),      # 168 whole K-sliced 64x64 tiles 36.5 us, 42 of 128x128 in four 44.5
+    (2352, 256, 3784, 256, True),      # 30.5 and 35.1
+    (75, 6624, 6144, 6624, True),      # 54.9 and 65.3
+    (444, 2304, 15360, 2304, False),   # deep: 110 whole, 85 split
+    (128, 4096, 16384, 4096, False),
+])
+def test_basic_down_keeps_one_wave_of_sliced_tiles(m, k, h, n, whole):
+    """A split of larger tiles has to beat one wave of whole K-sliced 64x64 tiles, which are priced too
+    high, by a margin below a depth of 9216."""
+    p = problem_from_shapes((m, k), (h, k), (n, h), "bfloat16")
+    native = make_plan(p, Selection("basic", "basic"), 256, tuned=False).native
+    assert (native.down_sk_tiles == 0) == whole
+    assert not whole or (native.down_bm, native.down_bn) == (64, 64)
 
 
 def test_swiglu_up_takes_narrow_tiles_at_small_m():
