@@ -442,9 +442,9 @@ bool swiglu_tile(const Variant& v) { return (v.bn / v.wgn) % 64 == 0; }
 
 // A tile that would be split competes only when no tiling of 64x64 or more fills more than half
 // of the grid with whole tiles: at 128 rows (128 x 4096 -> 16384) the 128x128 tile split in two
-// pieces priced ahead of 256 whole 64x128 tiles and measured 9-15% slower on the FFN; at 64 rows
-// and H 8192 only the 32x32 decode tiles fill the grid, and the split 64x64 tile stays 10%
-// ahead of them.
+// pieces priced ahead of 256 whole 64x128 tiles and takes 47.6 us, the whole ones 38.6 (256 x 2048 ->
+// 8192: 18.6 and 15.1; 256 x 4096 -> 8192 the other way, 32.7 and 33.6); at 64 rows and H 8192 only the
+// 32x32 decode tiles fill the grid, 12.5 us, and the split 64x64 tile takes 10.4.
 //
 // Pieces that straddle tiles are priced as the down's (144 rows, 1070 -> 2304, 108 tiles of 64x64 in
 // two uneven pieces: FFN 22.5 us, whole 16.8).  SwiGLU's K-sliced 64x64 tile needs four iterations:
@@ -487,13 +487,17 @@ int fast_dma_for(int k) { return k <= kFastDmaMaxK ? 1 : 0; }
 // Rotated K ranges (GemmParams::rot_step).  Workgroups that walk K in step read their weight rows at
 // one K offset at a time; where the row pitch is a multiple of 4 KiB those addresses differ in
 // their high bits alone, and they crowd on some of the memory channels.  Starting every tile
-// column at a place of its own in its K range spreads them.  Weights streamed from HBM, rotated
-// against in step, one run: 16 rows, 4096 -> 16384 -> 4096: up 31.0 -> 25.0 us, split down 32.3 ->
-// 27.8; 16 rows, 8192 x 8192: up 30.3 -> 26.9, down 29.6 -> 26.5; 128 rows, 4096 -> 16384: up 41.2 ->
-// 37.9, down 45.2 -> 42.9.  Pitches that are no such multiple (5120, 13824) and weights that stay in
-// the last-level cache are level or, on the shortest launches, 1% behind: they stay in step.  So do
-// taller problems, whose activation panel is shared in the L2 only while it is in step (4096 rows,
-// 1024 -> 4096: down 30.1 -> 42.6 us rotated).  The rule reads the padded widths, so that operands
+// column at a place of its own in its K range spreads them.  In step against rotated, the lines of
+// the rule on both sides (one run, eight shapes by nine row counts, the tiles of the automatic plans):
+//   weights, 1 to 128 rows: 128 MiB up 1.06-1.24, down 1.06-1.15 times faster (16 rows, 4096 -> 16384 ->
+//   4096: up 30.9 -> 24.9 us, split down 31.3 -> 27.4); 96 MiB 1.03-1.17; 64, 48 and 32 MiB 0.99-1.05,
+//   most of them within 2%: the gain ends about the line;
+//   rows, 96 and 128 MiB: 192 and 256 rows 1.04-1.07 where the tile is at most 64 rows tall (256 rows,
+//   6144 -> 8192 up 57.9 -> 54.5; taller tiles never rotate); 320 to 1024 rows 0.99-1.02, all but one of
+//   them on taller tiles; at 4096 rows the activation panel is shared in the L2 only in step
+//   (1024 -> 4096: down 30.1 -> 42.6 rotated).
+// Pitches that are no such multiple (5120, 13824) are level or, on the shortest launches, 1% behind.
+// The rule reads the padded widths, so that operands
 // read in place sum in the same order as their padded copies.
 constexpr int kRotMaxRows = 256;
 constexpr int kRotPitch = 4096;                // bytes
