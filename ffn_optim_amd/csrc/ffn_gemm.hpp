@@ -70,7 +70,7 @@ struct GemmParams {
     int group_m;          // tile-order swizzle: tiles walk group_m tile-rows column by column
     int fast_dma;         // 1: launch the kernel whose interior tiles refill through the SALU-addressed DMA path
     int rev_m;            // 1: tile rows are walked last-first
-    unsigned rot_step;    // tile column tn starts its K range tn * rot_step / 2^16 iterations in (TileCfg::ROT tiles)
+    unsigned rot_step;    // tile column tn starts its K range tn * rot_step / 2^16 iterations in (Rotated tiles)
     int zero_row0;        // rows [zero_row0, M) of C lie past every tile holding data: written as zeros
     int c_cols;           // columns of C (N, or N / 2 for SwiGLU, whose column pairs make one output)
     const void* bias;     // per-column bias in the storage type, added in FP32 before the activation
@@ -156,10 +156,10 @@ struct TileCfg {
     // after the previous iteration's stage barrier -- the moment the stage they fill is free --
     // instead of in the iteration before the data is used: a full iteration of lead for them.
     static constexpr int EARLY = EARLY_;
-    // Tiles whose units may take their K range rotated (Engine::first_kit): those of small-M GEMMs.
-    // (The wrap's three scalar instructions an iteration would cost the K-sliced 128x128 tile 0.5% on
-    // the aligned mid-size FFN.)
-    static constexpr bool ROT = BM_ <= 64;
+    // Tiles with a form whose units take their K range rotated (Rotated below, Engine::first_kit):
+    // those of small-M GEMMs.
+    static constexpr bool CAN_ROT = BM_ <= 64;
+    static constexpr bool ROT = false;
     static_assert(EARLY_ == 0 || (STAGES_ == 2 && WGK_ == 1 && EARLY_ < A_PW + B_PW),
                   "early refill: two stages, no K slices, part of the refill");
     static constexpr int LDS_BYTES = STAGES * STAGE_BYTES;
@@ -199,6 +199,16 @@ struct TileCfg {
     static_assert(SWZ_PERIOD == 1 || (A_PW % SWZ_PERIOD == 0 && B_PW % SWZ_PERIOD == 0),
                   "the swizzle phase of every DMA instruction must be known at compile time");
     static_assert(LDS_ALLOC <= LDS_MAX && LDS_USE <= LDS_MAX, "gfx950 has 160 KiB of LDS per CU");
+};
+
+// The form of a tile whose units take their K range rotated: a kernel of its own, launched where the
+// host asks for rotation.  In one kernel for both, the wrap's scalar instructions in every refill
+// cost the GEMMs that stay in step up to 9% (512x1024 -> 4096: v5 up 8.5 -> 8.9 us, v9 down
+// 18.8 -> 20.7; 624x6656 -> 2304: v5 up 36.7 -> 37.8, v14 42.0 -> 44.2).
+template <class C>
+struct Rotated : C {
+    static_assert(C::CAN_ROT, "tiles of small-M GEMMs");
+    static constexpr bool ROT = true;
 };
 
 // ---------------------------------------------------------------------------
@@ -558,8 +568,8 @@ struct Engine {
         }
         return d;
     }
-    // First K-iteration of a unit.  Tiles with C::ROT may take their range rotated, from a start in
-    // [kb, ke) on and wrapping at ke: tile columns start evenly spread, so that concurrent
+    // First K-iteration of a unit.  A Rotated tile takes its range from a start in [kb, ke) on,
+    // wrapping at ke: tile columns start evenly spread, so that concurrent
     // workgroups read their weight rows at different offsets (GemmParams::rot_step, 0: in order;
     // the host divides, which here cost a short launch 1.5%).  Tiles of one column share the start:
     // their panel of B is fetched once.

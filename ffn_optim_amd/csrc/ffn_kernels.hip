@@ -27,9 +27,11 @@ using Cfg = VariantCfg<FFN_VARIANT>::type;
 #define FFN_LAUNCHER FFN_CAT(ffn_launch_d, FFN_DT, _v, FFN_VARIANT)
 
 namespace {
-// one launch of ffn_gemm_kernel with the DMA addressing the plan chose
+// one launch of ffn_gemm_kernel with the K order and the DMA addressing the plan chose
 template <class CFG, int EPI, bool SK>
 void launch_gemm(const ffn::GemmParams* p, dim3 g, dim3 b, hipStream_t stream) {
+    if constexpr (CFG::CAN_ROT && !CFG::ROT)
+        if (p->rot_step) return launch_gemm<ffn::Rotated<CFG>, EPI, SK>(p, g, b, stream);
     if constexpr (EPI != ffn::EPI_STORE) {
         // up roles may read gathered activation rows
         if (p->a_gather) {
