@@ -26,6 +26,7 @@
 // across lanes into 16-byte stores.
 #pragma once
 
+#include <cstddef>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -70,7 +71,6 @@ struct GemmParams {
     int group_m;          // tile-order swizzle: tiles walk group_m tile-rows column by column
     int fast_dma;         // 1: launch the kernel whose interior tiles refill through the SALU-addressed DMA path
     int rev_m;            // 1: tile rows are walked last-first
-    unsigned rot_step;    // tile column tn starts its K range tn * rot_step / 2^16 iterations in (Rotated tiles)
     int zero_row0;        // rows [zero_row0, M) of C lie past every tile holding data: written as zeros
     int c_cols;           // columns of C (N, or N / 2 for SwiGLU, whose column pairs make one output)
     const void* bias;     // per-column bias in the storage type, added in FP32 before the activation
@@ -86,7 +86,12 @@ struct GemmParams {
     // the one that counts on it.
     unsigned* clear_words;
     int clear_count;
+    // Tile column tn of a Rotated tile starts its K range tn * rot_step / 2^16 iterations in.  Last, where
+    // the struct had padding: ahead of zero_row0 it moved the arguments behind it, and every kernel
+    // read them with one scalar load more.
+    unsigned rot_step;
 };
+static_assert(offsetof(GemmParams, rot_step) + sizeof(unsigned) == sizeof(GemmParams), "rot_step fills the padding");
 
 // Counter words of a single-launch FFN (ffn_fused.hip), in the workspace's counter region; zero
 // between launches (the last workgroup to leave clears them) but for the error word.  Each
