@@ -489,12 +489,12 @@ int fast_dma_for(int k) { return k <= kFastDmaMaxK ? 1 : 0; }
 // their high bits alone, and they crowd on some of the memory channels.  Starting every tile
 // column at a place of its own in its K range spreads them.  In step against rotated, the lines of
 // the rule on both sides (one run, eight shapes by nine row counts, the tiles of the automatic plans):
-//   weights, 1 to 128 rows: 128 MiB up 1.06-1.24, down 1.06-1.15 times faster (16 rows, 4096 -> 16384 ->
-//   4096: up 30.9 -> 24.9 us, split down 31.3 -> 27.4); 96 MiB 1.03-1.17; 64, 48 and 32 MiB 0.99-1.05,
-//   most of them within 2%: the gain ends about the line;
-//   rows, 96 and 128 MiB: 192 and 256 rows 1.04-1.07 where the tile is at most 64 rows tall (256 rows,
-//   6144 -> 8192 up 57.9 -> 54.5; taller tiles never rotate); 320 to 1024 rows 0.99-1.02, all but one of
-//   them on taller tiles; at 4096 rows the activation panel is shared in the L2 only in step
+//   weights, 1 to 128 rows: 128 MiB up 1.07-1.26, down 1.06-1.16 times faster (16 rows, 4096 -> 16384 ->
+//   4096: up 31.0 -> 24.8 us, split down 31.8 -> 27.9); 96 MiB 1.02-1.17; 64 MiB 0.95-1.06, 1.01 on
+//   average; 48 and 32 MiB 0.95-1.06, 1.01 on average: the gain ends about the line;
+//   rows, 96 and 128 MiB: 192 and 256 rows 1.02-1.06 where the tile is at most 64 rows tall (256 rows,
+//   6144 -> 8192 up 58.2 -> 54.7; taller tiles never rotate); 320 rows 1.00-1.01, 32 MiB at 320 rows
+//   0.97-1.00; at 4096 rows the activation panel is shared in the L2 only in step
 //   (1024 -> 4096: down 30.1 -> 42.6 rotated).
 // Pitches that are no such multiple (5120, 13824) are level or, on the shortest launches, 1% behind.
 // The rule reads the padded widths, so that operands
