@@ -743,3 +743,38 @@ def test_single_launch_with_an_automatic_down_tile():
     torch.cuda.synchronize()
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
     assert_parity(got, x, w1, w2, tag="single launch, automatic down")
+
+
+@pytest.mark.parametrize("activation", ["gelu", "swiglu"])
+def test_one_shot_call_captured_in_a_graph(activation):
+    """A one-shot call waits for nothing, so it can be captured: replayed on other inputs, with eager
+    work and synchronisations between the replays, it gives the eager results.  Odd widths (every operand
+    is staged) and a down whose tiles are split."""
+    from ffn_optim_amd import eagle_ffn_linear
+    m, k, h, n = 37, 999, 6161, 511
+    u = 2 * h if activation == "swiglu" else h
+    gen = torch.Generator(device="cuda").manual_seed(37)
+    shapes = ((m, k), (u, k), (n, h), (u,), (n,))
+    inputs = [[(torch.randn(s, generator=gen, device="cuda") * 0.03).bfloat16() for s in shapes] for _ in range(4)]
+    want = [eagle_ffn_linear(*t, activation).clone() for t in inputs]
+    static = [t.clone() for t in inputs[0]]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        eagle_ffn_linear(*static, activation)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    say("captured one-shot", activation)
+    with torch.cuda.graph(graph):
+        out = eagle_ffn_linear(*static, activation)
+    for replay in range(6):
+        i = replay % 4
+        for s, t in zip(static, inputs[i]):
+            s.copy_(t)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), want[i].view(torch.int16)), replay
+        again = eagle_ffn_linear(*inputs[(i + 1) % 4], activation)
+        torch.cuda.synchronize()
+        assert torch.equal(again.view(torch.int16), want[(i + 1) % 4].view(torch.int16)), replay
