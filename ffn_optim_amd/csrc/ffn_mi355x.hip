@@ -277,13 +277,18 @@ double cost_streamk(const Variant& v, const SkShape& s, long long m_valid, long 
     // pieces: 2.9 us for 16 KiB tiles, 5.4 for 64, 13.5 for 256; two pieces: 2.0 and 4.2 us for 16
     // and 64), many the memory traffic of the partials (128 tiles of 256x192 in two pieces: 75 MB
     // in 31 us; 64 of 256x256 in four: 117 MB in 38-46); pieces that straddle tiles finish two.
+    // Scattered pieces finish at different times, beside other workgroups' main loops: no traffic
+    // term.  (Priced with it, 60% over what 124 of them took, they lost to tiles that ran longer: 5616
+    // rows, 768 -> 2496, FFN 46.1 -> 52.9 us, 2016 rows, 528 -> 6656, 47.5 -> 53.0.  Over 70 FFNs whose
+    // pick this moves 1.03 times faster on average, 0.81 to 1.36.)
     // (the former prices count a piece more where the grid cuts every tile alike)
     const long long pieces_per_tile = s.pieces && !former
         ? s.pieces : std::min<long long>(G, cdiv(s.k_iters, std::max<long long>(1, s.q)) + 1);
     if (s.k_iters > sk_iters) {
         const double p = (double)pieces_per_tile;
         const double traffic = (double)s.sk * (2.0 * p - 1.0) * (double)v.bm * v.bn * 4.0 / kPartialRate;
-        t += former ? finish_latency(v, p, true) : std::max(finish_latency(v, p) * (scattered ? 2.0 : 1.0), traffic);
+        t += former ? finish_latency(v, p, true)
+                    : scattered ? 2.0 * finish_latency(v, p) : std::max(finish_latency(v, p), traffic);
     }
     const double hbm = (double)(N * K + m_valid * K) * 2.0 / kHbmRate;
     return std::max(t, hbm);

@@ -900,7 +900,7 @@ def test_known_plans_do_not_change_what_make_plan_accepts():
 @pytest.mark.parametrize("m, k, h, n, even", [
     (176, 2560, 3657, 2560, 14),     # 58 iterations of 64 in two; 29 of 128 do not halve
     (496, 4992, 863, 512, 14),
-    (1699, 1984, 1800, 4167, 6),     # 58 of 32 against 29 of 64
+    (128, 1762, 1359, 1762, 14),
 ])
 def test_streamk_pick_prefers_even_pieces(m, k, h, n, even):
     """Among near ties the automatic Stream-K down takes the tile whose pieces cut its iterations evenly."""
@@ -956,6 +956,15 @@ def test_basic_down_keeps_one_wave_of_sliced_tiles(m, k, h, n, whole):
     native = make_plan(p, Selection("basic", "basic"), 256, tuned=False).native
     assert (native.down_sk_tiles == 0) == whole
     assert not whole or (native.down_bm, native.down_bn) == (64, 64)
+
+
+@pytest.mark.parametrize("m, h, n", [(4160, 768, 7168), (1169, 1096, 3584), (2016, 528, 6656), (5616, 768, 2496)])
+def test_scattered_streamk_pieces_are_not_priced_for_traffic(m, h, n):
+    """Split tiles that do not divide the grid finish at different times: their partials overlap other
+    workgroups' main loops, and the 256x128 tile with refill waves stays the pick."""
+    plan = _c_plan(m, 64, h, n, "streamk")
+    assert (plan.down_bm, plan.down_bn) == (256, 128) and plan.down_grid == 256
+    assert 256 % plan.down_sk_tiles != 0
 
 
 def test_swiglu_up_takes_narrow_tiles_at_small_m():
