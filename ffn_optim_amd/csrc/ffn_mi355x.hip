@@ -454,8 +454,11 @@ bool swiglu_tile(const Variant& v) { return (v.bn / v.wgn) % 64 == 0; }
 // Pieces that straddle tiles are priced as the down's (144 rows, 1070 -> 2304, 108 tiles of 64x64 in
 // two uneven pieces: FFN 22.5 us, whole 16.8).  SwiGLU's K-sliced 64x64 tile needs four iterations:
 // on fewer the exchange of its slices is not made up for (490 rows, 256 -> 592: FFN 12.2 us, on the
-// 64x128 tile 11.5; 112 rows, 512 deep: level; 1024 deep: 7.7 against 8.3).
-constexpr long long kSlicedSwigluMinK = 512;
+// 64x128 tile 11.5; 112 rows, 512 deep: level; 1024 deep: 7.7 against 8.3).  With more than 64 rows
+// it competes with the 64x128 tile rather than the 128x128 one, and needs a K of 608: 512 to 564 deep the
+// FFNs of 128 to 783 rows took 2-5% longer on it (268 rows, 512 -> 1035: 13.0 and 13.7 us), 618 to 656 deep
+// they were 0-4% faster; up to 64 rows 512 deep and more 3-17% faster.
+constexpr long long kSlicedSwigluMinK = 512, kSlicedSwigluTallMinK = 608;
 int pick_up(long long M, long long m_valid, long long N, long long K, int G, bool swiglu) {
     int best = -1;
     double best_cost = 1e300;
@@ -465,7 +468,9 @@ int pick_up(long long M, long long m_valid, long long N, long long K, int G, boo
                  cdiv(m_valid, kVariants[i].bm) * cdiv(N, kVariants[i].bn) * 2 > G;
     for (int i = 0; i < kNumVariants; ++i) {
         if (swiglu && !swiglu_tile(kVariants[i])) continue;
-        if (swiglu && kVariants[i].wgk > 1 && kVariants[i].bm < 128 && K < kSlicedSwigluMinK) continue;
+        if (swiglu && kVariants[i].wgk > 1 && kVariants[i].bm < 128 &&
+            K < (m_valid > 64 ? kSlicedSwigluTallMinK : kSlicedSwigluMinK))
+            continue;
         SkShape s;
         const bool split = !swiglu && split_whole(kVariants[i], m_valid, N, K, G, s);
         if (split && fills) continue;

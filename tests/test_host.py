@@ -975,3 +975,6 @@ def test_swiglu_up_takes_narrow_tiles_at_small_m():
     assert (pick(16, 2048, 5504).up_bm, pick(16, 2048, 5504).up_bn) == (64, 64)
     assert pick(16, 4096, 11008).up_bm == 64
     assert pick(128, 4096, 11008).up_bm == 128
+    # shallow: up to 64 rows only (32 rows, 512 -> 1280 10% faster, 268 rows, 512 -> 1088 5% slower)
+    assert (pick(32, 512, 1280).up_variant, pick(268, 512, 1088).up_variant) == (16, 5)
+    assert pick(163, 640, 1536).up_variant == 16
